@@ -90,7 +90,14 @@ int Sequence::alloc(uint64_t bytes, void **out) {
   void *p = nullptr;
   if (hipMalloc(&p, bytes ? bytes : 256) != hipSuccess)
     return fail(BCH_ERR_ALLOCATION, "cannot allocate %llu bytes", (unsigned long long)bytes);
-  if (hipMemset(p, 0, bytes ? bytes : 256) != hipSuccess) return fail(BCH_ERR_ALLOCATION, "cannot clear memory");
+  // The clear runs on the null stream, which the model's (non-blocking)
+  // stream does not wait for: it must be done before a kernel writes the
+  // buffer (the weight expansions come right after their allocation, and a
+  // late clear zeroed some of what they wrote).
+  if (hipMemset(p, 0, bytes ? bytes : 256) != hipSuccess || hipStreamSynchronize(nullptr) != hipSuccess) {
+    hipFree(p);
+    return fail(BCH_ERR_ALLOCATION, "cannot clear memory");
+  }
   allocations.push_back(p);
   *out = p;
   return BCH_OK;
