@@ -142,12 +142,11 @@ constexpr uint32_t kMoeMaxUsed = 8;       // MOE_MAX_USED
 // Batched experts (prefill): grouping, grouped GEMM, weighted combine.
 void run_moe_group(hipStream_t s, const uint32_t *route, uint32_t *offsets, uint32_t *entries, uint32_t n_experts,
                    uint32_t n_used, uint32_t n_tokens);
-// split_ready (shared_input only): `split` already holds x's fp16 inputs
-// (run_rms_norm_split wrote them), so they are not converted again.
+// `split` holds matmul_expert_bytes(n_used·n_tokens, n_cols) bytes.
 void run_matmul_experts(hipStream_t s, uint32_t format, const uint8_t *W, const uint8_t *up, uint32_t n_rows,
                         uint32_t n_cols, uint32_t n_experts, const float *x, bool shared_input,
                         const uint32_t *offsets, const uint32_t *entries, uint32_t n_used, float *y,
-                        uint32_t n_tokens, void *split, bool split_ready = false);
+                        uint32_t n_tokens, void *split);
 void run_moe_combine(hipStream_t s, const float *x, const uint32_t *route, float *y, uint32_t n_embd,
                      uint32_t n_used, uint32_t n_tokens);
 // With `scores` (n_tokens · n_experts floats of scratch) and `counters`
@@ -305,6 +304,8 @@ uint64_t attn_prefill_partial_floats(uint32_t n_queries, uint32_t n_heads, uint3
 // launch may use (matmul_scratch_bytes(n_tokens, n_cols, n_rows) allows
 // all; matmul_split_bytes alone allows none).
 uint64_t matmul_split_bytes(uint32_t n_rows, uint32_t n_cols);
+// The grouped inputs of run_matmul_experts: `positions` rows of n_cols.
+uint64_t matmul_expert_bytes(uint32_t positions, uint32_t n_cols);
 uint64_t matmul_scratch_bytes(uint32_t n_tokens, uint32_t n_cols, uint32_t n_rows);
 // A column-split sum an accumulating run_matmul left for the next kernel:
 // y += Σ_split part[split] (n floats each), in split order.
@@ -320,8 +321,9 @@ void finish_pending_sum(hipStream_t s, PendingSum &p, float *y);
 // scratch, ..., split_ready = true) reads.  With `pending` (left by the
 // run_matmul that accumulated into x, on the same scratch) x first
 // receives that sum, written back to x; the pending sum is then cleared.
-// unscale_copy (optional, [rows]): a second copy of the token scales,
-// outside the scratch (run_blas_pair's).
+// unscale_copy (optional, [rows]): for run_blas_pair, a second copy of the
+// token scales outside the scratch, and the fp16 inputs as plain rows (a
+// run_matmul that follows instead converts its own).
 void run_rms_norm_split(hipStream_t s, float *x, const float *w, float *out, uint32_t n, uint32_t rows, float eps,
                         void *scratch, PendingSum *pending = nullptr, float *unscale_copy = nullptr);
 // store 3: y = silu(W·x) ⊙ (W2·x), W and W2 the gate and up matrices of

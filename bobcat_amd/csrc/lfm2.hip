@@ -314,7 +314,6 @@ static void lfm2_batch(bch_lfm2 *m, hipStream_t s, uint32_t pos, uint32_t count,
                  nullptr, defer);
       check_finite(s, "attn_output", il, m->hidden, (uint64_t)count * n);
     }
-    // (The MoE experts' shared input is this norm's output too.)
     const bool pair_ok = L.gate_up16 && count > kBlasPairMinTokens;
     run_rms_norm_split(s, m->hidden, L.ffn_norm, m->normed, n, count, m->norm_eps, m->split, &pend,
                        pair_ok ? m->pair_us : nullptr);
@@ -331,7 +330,7 @@ static void lfm2_batch(bch_lfm2 *m, hipStream_t s, uint32_t pos, uint32_t count,
         run_moe_group(s, m->route, m->moe_offsets, m->moe_entries, m->n_experts, m->n_used, count);
         run_matmul_experts(s, L.gate_exps.format, L.gate_exps.data, L.up_exps.data, m->n_ff_expert, n,
                            m->n_experts, m->normed, true, m->moe_offsets, m->moe_entries, m->n_used, m->expert_ffn,
-                           count, m->split, true);
+                           count, m->split);
         run_matmul_experts(s, L.down_exps.format, L.down_exps.data, nullptr, n, m->n_ff_expert, m->n_experts,
                            m->expert_ffn, false, m->moe_offsets, m->moe_entries, m->n_used, m->expert_out, count,
                            m->split);
@@ -350,7 +349,7 @@ static void lfm2_batch(bch_lfm2 *m, hipStream_t s, uint32_t pos, uint32_t count,
       if (!blas_pair && L.gate.format == L.up.format) {
         // Gate and up in one paired launch: ffn = silu(gate·x) ⊙ (up·x).
         run_matmul(s, L.gate.format, L.gate.data, m->n_ff, n, m->normed, m->ffn, count, 3, m->split, m->split_bytes,
-                   true, L.up.data);
+                   !pair_ok, L.up.data);
       } else if (!blas_pair) {
         run_matmul(s, L.gate.format, L.gate.data, m->n_ff, n, m->normed, m->ffn, count, 0, m->split, m->split_bytes,
                    true);
@@ -528,7 +527,7 @@ int bch_lfm2_new(bch_ctx *ctx, const bch_lfm2_model *md, uint32_t n_ctx, int kv_
     const uint32_t widest = std::max({n, m->q_dim, m->n_ff});
     const uint64_t split_bytes = m->split_bytes =
         std::max(matmul_scratch_bytes((uint32_t)rows, widest, n),
-                 matmul_split_bytes((uint32_t)(std::max(1u, m->n_used) * rows), std::max(1u, m->n_ff_expert)));
+                 any_moe ? matmul_expert_bytes((uint32_t)(m->n_used * rows), std::max(n, m->n_ff_expert)) : 0);
     int rc = 0;
     (void)((rc = m->alloc(cache, &m->k_cache)) || (rc = m->alloc(cache, &m->v_cache)) ||
            (rc = m->alloc_t((uint64_t)m->n_conv * (m->conv_kernel - 1) * n, &m->conv_state)) ||

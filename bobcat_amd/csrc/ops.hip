@@ -11,6 +11,7 @@
 #include <cmath>
 
 #include "formats.h"
+#include "frag.h"
 #include "kernels.h"
 #include "runtime.h"
 
@@ -327,10 +328,11 @@ __global__ __launch_bounds__(kConvThreads) void k_short_conv_split(const float *
     const int k2 = max(-100, min(100, 14 - ex));
     const float scale = ldexpf(1.0f, k2);
     if (tid == 0) unscale[tok] = ldexpf(1.0f, -k2);
+    const FragRow row = FragRow::of(H, tok, n_tokens, (n_embd + 7) / 8 * 8);
 #pragma unroll
     for (int c = 0; c < CPT; c++) {
       const uint32_t ch = tid + NT * c;
-      if (ch < n_embd) H[(uint64_t)tok * n_embd + ch] = (_Float16)(v[c][j] * scale);
+      if (ch < n_embd) *row.at(ch) = (_Float16)(v[c][j] * scale);
     }
   }
 }
@@ -585,7 +587,7 @@ bool run_short_conv_split(hipStream_t s, const float *bcx, const float *taps, fl
   // LFM2's convolutions have 3 taps; other sizes take the separate kernels.
   if (!n_tokens || ksize != 3 || n_embd == 0 || n_embd > 4 * kConvThreads) return false;
   _Float16 *hx = static_cast<_Float16 *>(scratch);
-  float *unscale = reinterpret_cast<float *>(hx + (uint64_t)n_tokens * n_embd);
+  float *unscale = reinterpret_cast<float *>(hx + (uint64_t)n_tokens * ((n_embd + 7) / 8 * 8));
   const uint32_t grid = div_ceil(n_tokens, kConvTokens);
   const uint32_t cpt = div_ceil(n_embd, kConvThreads);
   if (cpt <= 1)

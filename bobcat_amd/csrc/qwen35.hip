@@ -298,7 +298,7 @@ void bch_qwen35::record_batch(hipStream_t st, uint32_t pos, uint32_t count, bool
     const bool blas_pair = pair_ok && run_blas_pair(st, L.gate_up16, n_ff, n, count, split, pair_out, pair_us, nullptr);
     if (!blas_pair && L.gate.format == L.up.format) {
       // Gate and up in one paired launch: ffn = silu(gate·x) ⊙ (up·x).
-      run_matmul(st, L.gate.format, L.gate.data, n_ff, n, normed, ffn, count, 3, split, split_bytes, true,
+      run_matmul(st, L.gate.format, L.gate.data, n_ff, n, normed, ffn, count, 3, split, split_bytes, !pair_ok,
                  L.up.data);
     } else if (!blas_pair) {
       run_matmul(st, L.gate.format, L.gate.data, n_ff, n, normed, ffn, count, 0, split, split_bytes, true);
