@@ -3,17 +3,30 @@
 // its attention_flash kernel, crates/bobcat-metal/src/backend.rs:2150-2320,
 // attention.metal:289-480).
 //
-// One workgroup per (32 consecutive queries, KV head); wave w owns query
-// head kv·G + w of that KV head (G ≤ 4 query heads per KV head), so the four
-// waves share each key block's V tile in LDS.  Per block of 32 keys a wave
-// computes S^T = K·Q^T (keys × queries) with v_mfma_f32_32x32x16_f16, so each
-// lane holds 16 scores of one query: the online softmax needs one cross-lane
-// move (lane l and l^32 share a query), and the lane's accumulator registers
-// for keys 8j + 4·(l/32) + 0..3 are exactly the B operand of the next
-// product, O^T += V^T·P^T on v_mfma_f32_32x32x8_f16.  The queries and the
-// probabilities are split into f16 high and low parts (~22 bits) and both
-// are multiplied; K and V are the cache's f16 values, so the products are
-// exact and accumulate in f32.
+// A workgroup of four waves serves one KV head; a wave owns 32 consecutive
+// queries of one query head.  With a group of G query heads per KV head the
+// waves are G heads x 4/G query tiles (three heads leave one wave idle), so
+// they share every key block.  K and V of a block of 32 keys go to LDS once,
+// double buffered, the next block's loads in flight behind the current
+// block's MFMAs: reading K from the cache by each wave cost 32 cache lines
+// per load in four waves, more address cycles than the MFMAs take.
+//
+// Per block a wave computes S^T = K·Q^T (keys × queries) with
+// v_mfma_f32_32x32x16_f16, so each lane holds 16 scores of one query: the
+// online softmax needs one cross-lane move (lane l and l^32 share a query),
+// and the lane's scores of keys 16j + 4·(l/32) + {0..3, 8..11} are, as
+// probabilities, the B operand of k-step j of O^T += V^T·P^T; V is laid out
+// in LDS by quads of keys so that the A operand has the same keys.  The
+// queries and the probabilities are split into f16 high and low parts (~22
+// bits) and both are multiplied; K and V are the cache's f16 values, so the
+// products are exact and accumulate in f32.  Scores stay unscaled; the
+// softmax runs in powers of two, p = 2^(s·c − m), c = scale·log2(e).
+//
+// 512 queries over 8,192 keys, 32 x 8 heads of 64: 97 us with four key splits
+// and 9 us to combine them (340 TFLOP/s of the 4·hd operations a visible key
+// takes, the matrix cores doing twice that); 414 us before, unsplit.  What
+// bounds it now is issue slots: ~16 MFMAs and ~200 other instructions per
+// wave and block, most of them the softmax and the splitting of p.
 #include <algorithm>
 #include <cmath>
 
@@ -25,11 +38,13 @@ namespace bch {
 
 typedef _Float16 ph4_t __attribute__((ext_vector_type(4)));
 typedef _Float16 ph8_t __attribute__((ext_vector_type(8)));
+typedef _Float16 ph2_t __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+typedef float pf2_t __attribute__((ext_vector_type(2)));
 typedef float pf16_t __attribute__((ext_vector_type(16)));
 
-constexpr int kPrefQ = 32;        // queries per workgroup
+constexpr int kPrefQ = 32;        // queries per wave
 constexpr int kPrefKeys = 32;     // keys per block
-constexpr int kVtStride = 40;     // halves per V^T row in LDS (32 keys + padding)
 
 // The output gate of gated attention (Qwen3.5, qwen35.rs:422-424): with
 // `gate` set, output element d of (query z, head h) is multiplied by
@@ -42,31 +57,84 @@ struct AttnGate {
   }
 };
 
+// Query tiles per workgroup for a group of G query heads.
+__host__ __device__ constexpr uint32_t attn_prefill_tiles(uint32_t group) { return group == 1 ? 4 : group == 2 ? 2 : 1; }
+
 template <int HD>
-__global__ __launch_bounds__(256) void k_attn_prefill(const float *__restrict__ q, const _Float16 *__restrict__ kc,
+__global__ __launch_bounds__(256, HD == 64 ? 3 : HD == 128 ? 2 : 1) void k_attn_prefill(const float *__restrict__ q, const _Float16 *__restrict__ kc,
                                                       const _Float16 *__restrict__ vc, float *__restrict__ out,
                                                       uint32_t n_heads, uint32_t n_kv, uint32_t first_pos,
                                                       uint32_t n_queries, uint32_t q_stride, uint32_t out_stride,
                                                       float scale, float *__restrict__ partials, AttnGate gate) {
-  constexpr int KS = HD / 16;  // k-steps of the score product
-  constexpr int OB = HD / 32;  // 32-row blocks of the output
-  __shared__ _Float16 vt[HD * kVtStride];  // V^T of the current key block: [d][key]
+  constexpr int KS = HD / 16;      // k-steps of the score product
+  constexpr int OB = HD / 32;      // 32-row blocks of the output
+  constexpr int CH = HD / 8;       // 16-byte chunks of a cache row
+  constexpr int NP = HD / 64;      // pieces of K and of V per thread and block
+  // K: chunk c of key k at slot 32c + (k ^ c%8); V: keys 4i .. 4i+3 of
+  // element d at quad i·HD + d.
+  __shared__ __align__(16) _Float16 k_s[2][kPrefKeys * HD], v_s[2][kPrefKeys * HD];
   const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
-  const uint32_t kv = blockIdx.y, q0 = blockIdx.x * kPrefQ;
-  const uint32_t group = n_heads / n_kv;
-  const bool active = (uint32_t)wave < group;
-  const uint32_t head = kv * group + (active ? wave : 0);
+  const uint32_t kv = blockIdx.y, group = n_heads / n_kv, tiles = attn_prefill_tiles(group);
+  const uint32_t wg_q0 = blockIdx.x * tiles * kPrefQ;
+  const bool active = (uint32_t)wave < group * tiles && wg_q0 + wave / group * kPrefQ < n_queries;
+  const uint32_t head = kv * group + (active ? wave % group : 0);
+  const uint32_t q0 = wg_q0 + (active ? wave / group : 0) * kPrefQ;
   const uint32_t col = lane % 32, half_id = lane / 32;
   const uint32_t z = min(q0 + col, n_queries - 1);  // this lane's query (past the end: a copy, never stored)
   const uint32_t qpos = first_pos + q0 + col;
-  const uint32_t kend = first_pos + min(q0 + kPrefQ, n_queries);  // keys of the block's last query, exclusive
-  const uint64_t row_elems = (uint64_t)n_kv * HD;                 // cache elements per position
+  const uint32_t kend = first_pos + min(q0 + kPrefQ, n_queries);                      // keys of the wave's last query
+  const uint32_t wg_kend = first_pos + min(wg_q0 + tiles * kPrefQ, n_queries);        // and of the workgroup's
+  const uint64_t row_elems = (uint64_t)n_kv * HD;                                     // cache elements per position
   // Key split blockIdx.z of gridDim.z: a contiguous run of whole 32-key
-  // blocks of the tile's keys (possibly none, or none visible to a query:
-  // that split's partial then has max -inf and sum 0, and weighs nothing in
-  // the combine).
-  const uint32_t n_blocks = (kend + kPrefKeys - 1) / kPrefKeys, n_split = gridDim.z, split = blockIdx.z;
-  const uint32_t kb_lo = split * n_blocks / n_split * kPrefKeys, kb_hi = (split + 1) * n_blocks / n_split * kPrefKeys;
+  // blocks of the workgroup's keys (possibly none, or none visible to a
+  // query: that split's partial then has max -inf and sum 0, and weighs
+  // nothing in the combine).
+  const uint32_t n_blocks = (wg_kend + kPrefKeys - 1) / kPrefKeys, n_split = gridDim.z, split = blockIdx.z;
+  const uint32_t b_lo = (uint32_t)((uint64_t)split * n_blocks / n_split);
+  const uint32_t b_hi = (uint32_t)((uint64_t)(split + 1) * n_blocks / n_split);
+
+  // The block's cache rows through a descriptor of the block: rows past the
+  // end read zeros (their scores are masked), and an address is one constant
+  // per thread.
+  const uint32_t row_bytes = n_kv * HD * 2;
+  u32x4_t kr[NP];
+  uint32_t vr[NP][4];
+  auto load = [&](uint32_t blk) __attribute__((always_inline)) {
+    const uint32_t kb = blk * kPrefKeys, bytes = min((uint32_t)kPrefKeys, wg_kend - kb) * row_bytes - kv * HD * 2;
+    const uint64_t at = kb * row_elems + (uint64_t)kv * HD;
+    const __amdgpu_buffer_rsrc_t kd = __builtin_amdgcn_make_buffer_rsrc(const_cast<_Float16 *>(kc) + at, 0, bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t vd = __builtin_amdgcn_make_buffer_rsrc(const_cast<_Float16 *>(vc) + at, 0, bytes, 0x00020000);
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+      const uint32_t c = tid + 256 * p;
+      kr[p] = __builtin_amdgcn_raw_buffer_load_b128(kd, c / CH * row_bytes + (c % CH) * 16, 0, 0);
+    }
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+      const uint32_t c = tid + 256 * p, dp = c % (HD / 2), kq = c / (HD / 2);
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        vr[p][i] = __builtin_amdgcn_raw_buffer_load_b32(vd, 4 * kq * row_bytes + 4 * dp, i * row_bytes, 0);
+    }
+  };
+  auto stage = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+      const uint32_t c = tid + 256 * p, key = c / CH, chunk = c % CH;
+      *reinterpret_cast<u32x4_t *>(&k_s[buf][(chunk * 32 + (key ^ (chunk & 7))) * 8]) = kr[p];
+    }
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+      const uint32_t c = tid + 256 * p, dp = c % (HD / 2), kq = c / (HD / 2);
+      // (k0, k1) and (k2, k3) of elements 2dp (low halves) and 2dp + 1.
+      const u32x4_t w = {__builtin_amdgcn_perm(vr[p][1], vr[p][0], 0x05040100u),
+                       __builtin_amdgcn_perm(vr[p][3], vr[p][2], 0x05040100u),
+                       __builtin_amdgcn_perm(vr[p][1], vr[p][0], 0x07060302u),
+                       __builtin_amdgcn_perm(vr[p][3], vr[p][2], 0x07060302u)};
+      *reinterpret_cast<u32x4_t *>(&v_s[buf][(kq * HD + 2 * dp) * 4]) = w;
+    }
+  };
+  if (b_lo < b_hi) load(b_lo);
 
   // The query's k-step fragments as the B operand: Q[z][16·s + 8·half .. +8].
   ph8_t qh[KS], ql[KS];
@@ -84,130 +152,98 @@ __global__ __launch_bounds__(256) void k_attn_prefill(const float *__restrict__ 
       }
     }
   }
-
   pf16_t o[OB];
 #pragma unroll
   for (int b = 0; b < OB; b++)
 #pragma unroll
     for (int i = 0; i < 16; i++) o[b][i] = 0.f;
-  float m_run = -INFINITY, l_run = 0.f;
+  float m_run = -INFINITY, l_run = 0.f;  // the maximum in units of log2
+  const float c2 = scale * 1.44269504088896340736f;
 
-  // Key block kb's loads: this thread's VP pieces of V (8 halves each,
-  // staged transposed in LDS) and this lane's K fragments, both with
-  // clamped rows (the staging zeroes V past kend; scores past it are
-  // masked).  Each block's loads are issued one block ahead, before the
-  // current block's MFMAs, so that the memory latency overlaps them
-  // (loading in the block itself put a full round trip on every block).
-  constexpr int VP = kPrefKeys * HD / 8 / 256;
-  static_assert(VP >= 1 && kPrefKeys * HD / 8 == 256 * VP, "V pieces per thread");
-  auto load_v = [&](uint32_t kb, ph8_t *v8) __attribute__((always_inline)) {
-#pragma unroll
-    for (int p = 0; p < VP; p++) {
-      const uint32_t c = tid + 256 * p, key = c / (HD / 8), d0 = (c % (HD / 8)) * 8;
-      const uint32_t row = min(kb + key, kend - 1);
-      v8[p] = *reinterpret_cast<const ph8_t *>(vc + (uint64_t)row * row_elems + (uint64_t)kv * HD + d0);
-    }
-  };
-  auto load_k = [&](uint32_t kb, ph8_t *ka) __attribute__((always_inline)) {
-    const uint32_t krow = min(kb + col, kend - 1);
-    const _Float16 *kr = kc + (uint64_t)krow * row_elems + (uint64_t)kv * HD + 8 * half_id;
-#pragma unroll
-    for (int s = 0; s < KS; s++) ka[s] = *reinterpret_cast<const ph8_t *>(kr + 16 * s);
-  };
-
-  // (Heads of 256 hold a 32 x 256 f32 output tile per wave in registers:
-  // they load each block in the block itself, as a second register set
-  // would not fit.)
-  constexpr bool kAhead = HD <= 128;
-  auto block = [&](uint32_t kb, const ph8_t *ka, const ph8_t *vcur, ph8_t *kn, ph8_t *vn)
-                   __attribute__((always_inline)) {
-    // Stage V^T of keys kb .. kb+31 (zeros past kend).
-    __syncthreads();
-#pragma unroll
-    for (int p = 0; p < VP; p++) {
-      const uint32_t c = tid + 256 * p, key = c / (HD / 8), d0 = (c % (HD / 8)) * 8;
-      const bool in = kb + key < kend;
-#pragma unroll
-      for (int j = 0; j < 8; j++) vt[(d0 + j) * kVtStride + key] = in ? vcur[p][j] : (_Float16)0.f;
-    }
-    __syncthreads();
-    // The next block's loads (a clamped re-read past the split's end).
-    if constexpr (kAhead) {
-      const uint32_t nb = min(kb + kPrefKeys, kb_hi - kPrefKeys);
-      load_v(nb, vn);
-      load_k(nb, kn);
-    }
-    if (!active) return;
-
+  auto block = [&](uint32_t kb, int buf) __attribute__((always_inline)) {
     // S^T = K·Q^T: lane supplies K[kb + col][16·s + 8·half .. +8].
     pf16_t sc;
 #pragma unroll
     for (int i = 0; i < 16; i++) sc[i] = 0.f;
 #pragma unroll
     for (int s = 0; s < KS; s++) {
-      sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka[s], qh[s], sc, 0, 0, 0);
-      sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka[s], ql[s], sc, 0, 0, 0);
+      const uint32_t chunk = 2 * s + half_id;
+      const ph8_t ka = *reinterpret_cast<const ph8_t *>(&k_s[buf][(chunk * 32 + (col ^ (chunk & 7))) * 8]);
+      sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka, qh[s], sc, 0, 0, 0);
+      sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka, ql[s], sc, 0, 0, 0);
     }
-    // sc[r] is the score of key kb + 8·(r/4) + 4·half + r%4 for this lane's query.
-    float mx = -INFINITY;
+    // sc[r] is the score of key kb + 8·(r/4) + 4·half + r%4 for this lane's
+    // query; only blocks that reach past the wave's first query have a key
+    // to mask.
+    if (kb + kPrefKeys - 1 > first_pos + q0) {
 #pragma unroll
-    for (int r = 0; r < 16; r++) {
-      const uint32_t key = kb + 8 * (r / 4) + 4 * half_id + (r % 4);
-      sc[r] = (key <= qpos && key < kend) ? sc[r] * scale : -INFINITY;
-      mx = fmaxf(mx, sc[r]);
+      for (int r = 0; r < 16; r++) {
+        const uint32_t key = kb + 8 * (r / 4) + 4 * half_id + (r % 4);
+        if (key > qpos || key >= kend) sc[r] = -INFINITY;
+      }
     }
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    float mx = sc[0];
+#pragma unroll
+    for (int r = 1; r < 16; r++) mx = fmaxf(mx, sc[r]);
+    // (The two lanes of a query, 32 apart: the swap leaves both values in each.)
+    const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+    mx = fmaxf(__uint_as_float(both[0]), __uint_as_float(both[1])) * c2;
     // -inf while no key of this split has been visible to the query (a
     // causal split can start after it): the block then adds exact zeros.
-    const float m_new = fmaxf(m_run, mx);
-    const float m_use = m_new == -INFINITY ? 0.f : m_new;
-    const float corr = expf(m_run - m_use);
-    m_run = m_new;
-    float psum = 0.f;
-    ph4_t ph[4], pl[4];
+    if (__builtin_amdgcn_ballot_w64(mx > m_run)) {
+      const float m_new = fmaxf(m_run, mx);
+      const float corr = m_new == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m_run - m_new);
+      m_run = m_new;
+      l_run *= corr;
 #pragma unroll
-    for (int r = 0; r < 16; r++) {
-      const float p = expf(sc[r] - m_use);
-      psum += p;
-      const _Float16 h = (_Float16)p;
-      ph[r / 4][r % 4] = h;
-      pl[r / 4][r % 4] = (_Float16)(p - (float)h);
+      for (int b = 0; b < OB; b++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) o[b][i] *= corr;
     }
-    l_run = l_run * corr + psum;
+    const float m_use = m_run == -INFINITY ? 0.f : m_run;
+    float psum = 0.f;
+    ph8_t ph[2], pl[2];
 #pragma unroll
-    for (int b = 0; b < OB; b++)
+    for (int r = 0; r < 16; r += 2) {
+      const float p0 = __builtin_amdgcn_exp2f(fmaf(sc[r], c2, -m_use));
+      const float p1 = __builtin_amdgcn_exp2f(fmaf(sc[r + 1], c2, -m_use));
+      psum += p0 + p1;
+      const pf2_t pv = {p0, p1};
+      const ph2_t hi = __builtin_convertvector(pv, ph2_t);
+      const pf2_t rest = {p0 - (float)hi[0], p1 - (float)hi[1]};
+      const ph2_t lo = __builtin_convertvector(rest, ph2_t);
+      ph[r / 8][r % 8] = hi[0], ph[r / 8][r % 8 + 1] = hi[1];
+      pl[r / 8][r % 8] = lo[0], pl[r / 8][r % 8 + 1] = lo[1];
+    }
+    l_run += psum;
+    // O^T += V^T·P^T over 2 k-steps of 16 keys: lane supplies V^T[32b + col]
+    // of keys 16j + 4·half + {0..3, 8..11} and the probabilities of the same.
 #pragma unroll
-      for (int i = 0; i < 16; i++) o[b][i] *= corr;
-    // O^T += V^T·P^T over 4 k-steps of 8 keys: lane supplies
-    // V^T[32b + col][8j + 4·half .. +4] and P^T[8j + 4·half .. +4][col].
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
+    for (int j = 0; j < 2; j++) {
 #pragma unroll
       for (int b = 0; b < OB; b++) {
-        const ph4_t a = *reinterpret_cast<const ph4_t *>(vt + (32 * b + col) * kVtStride + 8 * j + 4 * half_id);
-        o[b] = __builtin_amdgcn_mfma_f32_32x32x8f16(a, ph[j], o[b], 0, 0, 0);
-        o[b] = __builtin_amdgcn_mfma_f32_32x32x8f16(a, pl[j], o[b], 0, 0, 0);
+        const uint32_t d = 32 * b + col;
+        const ph4_t v0 = *reinterpret_cast<const ph4_t *>(&v_s[buf][((4 * j + half_id) * HD + d) * 4]);
+        const ph4_t v1 = *reinterpret_cast<const ph4_t *>(&v_s[buf][((4 * j + 2 + half_id) * HD + d) * 4]);
+        const ph8_t a = __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
+        o[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, ph[j], o[b], 0, 0, 0);
+        o[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, pl[j], o[b], 0, 0, 0);
       }
     }
   };
-  // Two register sets, alternating block by block.
-  const uint32_t kb_end = min(kb_hi, (kend + kPrefKeys - 1) / kPrefKeys * kPrefKeys);
-  if constexpr (kAhead) {
-    if (kb_lo < kb_end) {
-      ph8_t kA[KS], kB[KS], vA[VP], vB[VP];
-      load_v(kb_lo, vA);
-      load_k(kb_lo, kA);
-      for (uint32_t kb = kb_lo; kb < kb_end; kb += 2 * kPrefKeys) {
-        block(kb, kA, vA, kB, vB);
-        if (kb + kPrefKeys < kb_end) block(kb + kPrefKeys, kB, vB, kA, vA);
+  if (b_lo < b_hi) {
+    stage(0);
+    load(min(b_lo + 1, b_hi - 1));
+    lds_barrier();
+    for (uint32_t b = b_lo; b < b_hi; b++) {
+      const int buf = (int)((b - b_lo) & 1);
+      // Buffer buf ^ 1 was read before the last barrier.
+      if (b + 1 < b_hi) {
+        stage(buf ^ 1);
+        load(min(b + 2, b_hi - 1));
       }
-    }
-  } else {
-    for (uint32_t kb = kb_lo; kb < kb_end; kb += kPrefKeys) {
-      ph8_t kA[KS], vA[VP];
-      load_v(kb, vA);
-      if (active) load_k(kb, kA);
-      block(kb, kA, vA, nullptr, nullptr);
+      if (active && b * kPrefKeys < kend) block(b * kPrefKeys, buf);
+      lds_barrier();
     }
   }
   if (!active) return;
@@ -216,8 +252,8 @@ __global__ __launch_bounds__(256) void k_attn_prefill(const float *__restrict__ 
   float inv = 1.f / l_all;
   float *orow = out + (uint64_t)(q0 + col) * out_stride + (uint64_t)head * HD;
   if (n_split > 1) {
-    // Unnormalised partial (max, sum, output) of this split, combined by
-    // k_attn_prefill_combine.
+    // Unnormalised partial (max in log2, sum, output) of this split,
+    // combined by k_attn_prefill_combine.
     float *pp = partials + (((uint64_t)(q0 + col) * n_heads + head) * n_split + split) * (HD + 2);
     if (half_id == 0) {
       pp[0] = m_run;
@@ -255,7 +291,7 @@ __global__ __launch_bounds__(HD) void k_attn_prefill_combine(const float *__rest
   for (uint32_t sp = 0; sp < n_split; sp++) M = fmaxf(M, pp[sp * (HD + 2)]);
   float L = 0.f, O = 0.f;
   for (uint32_t sp = 0; sp < n_split; sp++) {
-    const float w = expf(pp[sp * (HD + 2)] - M);
+    const float w = __builtin_amdgcn_exp2f(pp[sp * (HD + 2)] - M);
     L = fmaf(pp[sp * (HD + 2) + 1], w, L);
     O = fmaf(pp[sp * (HD + 2) + 2 + d], w, O);
   }
@@ -274,11 +310,13 @@ uint64_t attn_prefill_partial_floats(uint32_t n_queries, uint32_t n_heads, uint3
 uint32_t attn_prefill_splits(uint32_t n_heads, uint32_t n_kv, uint32_t head_dim, uint32_t first_pos,
                              uint32_t n_queries, uint64_t partial_floats) {
   if (!n_queries) return 1;
-  // Enough workgroups for two per CU, at least kMinSplitBlocks 32-key blocks
+  // Enough workgroups for two per CU (three, which heads of 64 have registers
+  // for, made their kernel 4% faster and its combine as much slower), at least kMinSplitBlocks 32-key blocks
   // per split of the batch's middle tile, and no more partials than the
   // scratch holds.
   constexpr uint32_t kTargetGroups = 512, kMinSplitBlocks = 2, kMaxSplits = 16;
-  const uint32_t tiles = (n_queries + kPrefQ - 1) / kPrefQ;
+  const uint32_t per_wg = kPrefQ * attn_prefill_tiles(n_heads / n_kv);
+  const uint32_t tiles = (n_queries + per_wg - 1) / per_wg;
   uint32_t want = (kTargetGroups + tiles * n_kv - 1) / (tiles * n_kv);
   const uint32_t mid_blocks = (first_pos + (n_queries + 1) / 2 + kPrefKeys - 1) / kPrefKeys;
   want = std::min(want, mid_blocks / kMinSplitBlocks);
@@ -296,7 +334,8 @@ void run_attn_prefill_mfma(hipStream_t s, const float *q, const void *k_cache, c
   if (!n_queries) return;
   const uint32_t n_split =
       partials ? attn_prefill_splits(n_heads, n_kv, head_dim, first_pos, n_queries, partial_floats) : 1;
-  const dim3 grid((n_queries + kPrefQ - 1) / kPrefQ, n_kv, n_split);
+  const uint32_t per_wg = kPrefQ * attn_prefill_tiles(n_heads / n_kv);
+  const dim3 grid((n_queries + per_wg - 1) / per_wg, n_kv, n_split);
   const _Float16 *kc = static_cast<const _Float16 *>(k_cache);
   const _Float16 *vc = static_cast<const _Float16 *>(v_cache);
   const AttnGate g{gate, gate_head_stride, gate_query_stride};
@@ -340,9 +379,22 @@ extern "C" int bch_attention_prefill(bch_ctx *ctx, bch_view q, bch_view k_cache,
   if (reinterpret_cast<uintptr_t>(kp) % 16 || reinterpret_cast<uintptr_t>(vp) % 16 ||
       reinterpret_cast<uintptr_t>(qp) % 16 || reinterpret_cast<uintptr_t>(op) % 16)
     return fail(BCH_ERR_ARGUMENT, "attention_prefill: operands must be 16-byte aligned");
+  // Key splits with their partials in the context's scratch; without the
+  // memory for them the launch runs unsplit.
+  float *partials = nullptr;
+  uint64_t partial_floats = 0;
+  const uint32_t splits = n_queries ? attn_prefill_splits(n_heads, n_kv_heads, head_dim, first_pos, n_queries, ~0ull) : 1;
+  if (splits > 1) {
+    void *p = nullptr;
+    partial_floats = attn_prefill_partial_floats(n_queries, n_heads, head_dim, splits);
+    if (ctx_scratch(ctx, partial_floats * 4, &p) == BCH_OK)
+      partials = static_cast<float *>(p);
+    else
+      (void)hipGetLastError();
+  }
   return launch(ctx, {"attention_prefill", 0, 0, 0}, [&](hipStream_t s) {
     run_attn_prefill_mfma(s, qp, kp, vp, op, n_heads, n_kv_heads, head_dim, first_pos, n_queries,
-                          n_heads * head_dim, n_heads * head_dim, 1.0f / sqrtf((float)head_dim), nullptr, 0,
-                          nullptr, 0, 0);
+                          n_heads * head_dim, n_heads * head_dim, 1.0f / sqrtf((float)head_dim), partials,
+                          partial_floats, nullptr, 0, 0);
   });
 }
