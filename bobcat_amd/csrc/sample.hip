@@ -5,9 +5,11 @@
 // Steps, in the reference's (llama.cpp's) order:
 //   1. repetition penalty on each distinct token of the last 64, in place;
 //   2. temperature <= 0: argmax (ties to the lowest id);
-//   3. top-k: a radix select finds the k-th largest logit and a scan-based
-//      compaction keeps the k candidates (ties at the threshold by lowest
-//      id), at most kMaxCandidates of them;
+//   3. top-k: up to kFastTopK candidates, a bound that at least k of the
+//      threads' maxima reach keeps little more than the k largest logits,
+//      which are sorted and cut; else a radix select finds the k-th largest
+//      logit and a scan-based compaction keeps the k candidates (ties at the
+//      threshold by lowest id), at most kMaxCandidates of them;
 //   4. the candidates are sorted by logit (bitonic sort in LDS), then
 //      softmax at temperature 1, the top-p prefix, the min-p floor, log and
 //      softmax at the temperature, and a draw walking the sorted candidates.
@@ -16,6 +18,13 @@
 // sorted list (the top-p prefix and the draw) instead finds the rank where
 // the cumulative mass crosses its target by a radix descent over the logits'
 // ordered keys with mass histograms (sample_large below).
+//
+// One workgroup walks the logits, so what bounds it is one CU's load path
+// (64 bytes a cycle, ~2 us per pass over 65,536 logits) and the latencies
+// between passes: loads are issued eight at a time, nothing is scanned by a
+// single thread, and the top-k path reads the logits twice (155 us before,
+// 29 us now for 65,536 logits, top-k 40; with top_k = 0 and top-p 0.9 a pass
+// with its 8 us projection took 413 us and takes 189).
 // The draw comes from a wyrand generator whose 64-bit state lives in device
 // memory, so graph replays continue the stream.  Sums run as tree
 // reductions/scans instead of the reference's sequential loops, so draws
@@ -30,6 +39,25 @@ namespace bch {
 
 constexpr uint32_t kSampleThreads = 1024;
 constexpr uint32_t kRepeatLastN = 64;  // REPEAT_LAST_N (sampler.rs:8-9)
+// Top-k up to here takes the bound of the threads' maxima: with k of 1,024
+// maxima at or above it, ~-1024·ln(1 - k/1024) logits are (1,420 for 768).
+constexpr uint32_t kFastTopK = 768;
+
+// f(i, logits[i]) for the elements of this thread (i = tid, tid + 1024, ...),
+// eight loads in flight.
+template <class F>
+__device__ __forceinline__ void for_each_logit(const float *logits, uint32_t n, F f) {
+  constexpr int U = 8;
+  uint32_t i = threadIdx.x;
+  for (; i + (U - 1) * kSampleThreads < n; i += U * kSampleThreads) {
+    float v[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) v[u] = logits[i + u * kSampleThreads];
+#pragma unroll
+    for (int u = 0; u < U; u++) f(i + u * kSampleThreads, v[u]);
+  }
+  for (; i < n; i += kSampleThreads) f(i, logits[i]);
+}
 
 __device__ __forceinline__ uint32_t ord_key(float v) {
   uint32_t b = __float_as_uint(v);
@@ -226,7 +254,149 @@ __device__ Cut mass_cut(const float *logits, uint32_t n, uint64_t target, bool i
   return Cut{prefix, id};
 }
 
-__device__ void sample_large(const SampleArgs &a, uint32_t k, uint64_t *bins, uint32_t *u16, float *f16s,
+// The candidates of a list in LDS, in rank order: logit descending, id
+// ascending.  P (a power of two) entries, the unused ones (-inf, 0xffffffff).
+__device__ void sort_candidates(float *cval, uint32_t *cidx, uint32_t P) {
+  for (uint32_t size = 2; size <= P; size <<= 1) {
+    for (uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
+      for (uint32_t i = threadIdx.x; i < P; i += kSampleThreads) {
+        const uint32_t j = i ^ stride;
+        if (j > i) {
+          const bool desc = (i & size) == 0;
+          const float vi = cval[i], vj = cval[j];
+          const uint32_t ii = cidx[i], ij = cidx[j];
+          const bool i_first = vi > vj || (vi == vj && ii < ij);
+          if (desc != i_first) {
+            cval[i] = vj;
+            cval[j] = vi;
+            cidx[i] = ij;
+            cidx[j] = ii;
+          }
+        }
+      }
+      __syncthreads();
+    }
+  }
+}
+
+// Appends (v, i) of the lanes with `take` to the list, whatever its order
+// (the sort fixes it); *count may exceed kMaxCandidates, the excess is not
+// stored.
+__device__ __forceinline__ void append(bool take, float v, uint32_t i, float *cval, uint32_t *cidx, uint32_t *count) {
+  const uint64_t m = __builtin_amdgcn_ballot_w64(take);
+  if (!m) return;
+  const uint32_t lane = threadIdx.x % 64;
+  uint32_t base = 0;
+  const int lead = __ffsll((unsigned long long)m) - 1;
+  if ((int)lane == lead) base = atomicAdd(count, (uint32_t)__popcll(m));
+  base = __shfl(base, lead, 64);
+  const uint32_t at = base + (uint32_t)__popcll(m & ((1ull << lane) - 1));
+  if (take && at < kMaxCandidates) {
+    cval[at] = v;
+    cidx[at] = i;
+  }
+}
+
+constexpr uint32_t kMassBins = 4096;  // by the top 12 bits of a key: an eighth of an octave each
+struct SampleLds {
+  float cval[kMaxCandidates];
+  uint32_t cidx[kMaxCandidates];
+  uint64_t bins[kMassBins];
+  uint64_t s16[16];
+  uint32_t count, bin, low;
+  uint64_t above;
+};
+
+// mass_cut with one histogram pass over 4,096 bins and one pass that collects
+// the elements of the crossing bin, which are then ranked exactly.  The
+// weights are the same integers, so the cut is mass_cut's; more elements in
+// the bin than the list holds go to mass_cut.
+template <class Pred, class Weight>
+__device__ Cut mass_cut_list(const float *logits, uint32_t n, uint64_t target, bool inclusive, Pred pred, Weight weight,
+                             SampleLds &L, uint64_t *bins, uint32_t *u16, uint32_t *sel_s, uint64_t *above_s,
+                             bool *found) {
+  constexpr uint32_t kPer = kMassBins / kSampleThreads, kNone = 0xffffffffu;
+  const uint32_t tid = threadIdx.x;
+  for (uint32_t i = tid; i < kMassBins; i += kSampleThreads) L.bins[i] = 0;
+  if (tid == 0) L.bin = kNone, L.low = kNone, L.count = 0;
+  __syncthreads();
+  for_each_logit(logits, n, [&](uint32_t i, float v) {
+    if (pred(i, v))
+      atomicAdd(reinterpret_cast<unsigned long long *>(&L.bins[ord_key(v) >> 20]), (unsigned long long)mass_fixed(weight(v)));
+  });
+  __syncthreads();
+  // Thread t holds bins 4095 - 4t .. 4092 - 4t, the highest first.
+  uint64_t mine = 0;
+  const uint32_t top = kMassBins - 1 - kPer * tid;
+#pragma unroll
+  for (uint32_t k = 0; k < kPer; k++) mine += L.bins[top - k];
+  uint64_t total;
+  uint64_t acc = block_scan<uint64_t>(mine, L.s16, &total);
+#pragma unroll
+  for (uint32_t k = 0; k < kPer; k++) {
+    const uint64_t b = L.bins[top - k], next = acc + b;
+    const bool before = inclusive ? acc >= target : acc > target, after = inclusive ? next >= target : next > target;
+    // (A target of 0 is reached by the first bin with weight.)
+    if (b && after && (!before || acc == 0)) L.bin = top - k, L.above = acc;
+    if (b) atomicMin(&L.low, top - k);
+    acc = next;
+  }
+  __syncthreads();
+  const bool reached = L.bin != kNone;
+  const uint32_t bin = reached ? L.bin : L.low;
+  if (bin == kNone) {  // nothing passes the predicate
+    *found = false;
+    __syncthreads();
+    return Cut{0u, 0u};
+  }
+  const uint64_t above = reached ? L.above : total - L.bins[bin];
+  for_each_logit(logits, n, [&](uint32_t i, float v) {
+    append(ord_key(v) >> 20 == bin && pred(i, v), v, i, L.cval, L.cidx, &L.count);
+  });
+  __syncthreads();
+  const uint32_t m = L.count;
+  if (m > kMaxCandidates) {
+    __syncthreads();
+    return mass_cut(logits, n, target, inclusive, [&](uint32_t i) { return pred(i, logits[i]); }, weight, bins, u16, sel_s,
+                    above_s, found);
+  }
+  uint32_t P = 1;
+  while (P < m) P <<= 1;
+  for (uint32_t i = m + tid; i < P; i += kSampleThreads) {
+    L.cval[i] = -INFINITY;
+    L.cidx[i] = kNone;
+  }
+  __syncthreads();
+  sort_candidates(L.cval, L.cidx, P);
+  // The first rank whose cumulative weight crosses; without one, the last
+  // rank with any weight.
+  const uint32_t per = (m + kSampleThreads - 1) / kSampleThreads, lo = min(m, tid * per), hi = min(m, lo + per);
+  uint64_t part = 0;
+  for (uint32_t i = lo; i < hi; i++) part += mass_fixed(weight(L.cval[i]));
+  uint64_t sum;
+  uint64_t cum = above + block_scan<uint64_t>(part, L.s16, &sum);
+  if (tid == 0) L.low = reached ? kNone : 0;
+  __syncthreads();
+  for (uint32_t i = lo; i < hi; i++) {
+    const uint64_t w = mass_fixed(weight(L.cval[i]));
+    cum += w;
+    if (reached ? (w && (inclusive ? cum >= target : cum > target)) : w != 0) {
+      if (reached) {
+        atomicMin(&L.low, i);
+        break;
+      }
+      atomicMax(&L.low, i);
+    }
+  }
+  __syncthreads();
+  const uint32_t at = min(L.low, m - 1);
+  const Cut c{ord_key(L.cval[at]), L.cidx[at]};
+  *found = reached;
+  __syncthreads();
+  return c;
+}
+
+__device__ void sample_large(const SampleArgs &a, uint32_t k, SampleLds &L, uint64_t *bins, uint32_t *u16, float *f16s,
                              uint32_t *sel_s, uint64_t *above_s, uint32_t *token_s) {
   const uint32_t tid = threadIdx.x, n = a.n;
   const float *logits = a.logits;
@@ -234,58 +404,61 @@ __device__ void sample_large(const SampleArgs &a, uint32_t k, uint64_t *bins, ui
   Cut topk{0u, 0xffffffffu};
   if (k < n) {
     bool f;
-    topk = mass_cut(
-        logits, n, (uint64_t)k << 40, true, [](uint32_t) { return true; }, [](float) { return 1.0f; }, bins, u16,
-        sel_s, above_s, &f);
+    topk = mass_cut_list(
+        logits, n, (uint64_t)k << 40, true, [](uint32_t, float) { return true; }, [](float) { return 1.0f; }, L, bins,
+        u16, sel_s, above_s, &f);
   }
-  auto in_topk = [&](uint32_t i) { return before_cut(ord_key(logits[i]), i, topk); };
+  auto in_topk = [&](uint32_t i, float v) { return before_cut(ord_key(v), i, topk); };
   // 2. Softmax at temperature 1 over the candidates.
   float mx = -INFINITY;
-  for (uint32_t i = tid; i < n; i += kSampleThreads)
-    if (in_topk(i)) mx = fmaxf(mx, logits[i]);
+  for_each_logit(logits, n, [&](uint32_t i, float v) {
+    if (in_topk(i, v)) mx = fmaxf(mx, v);
+  });
   mx = block_max<kSampleThreads>(mx, f16s);
   float part = 0.f;
-  for (uint32_t i = tid; i < n; i += kSampleThreads)
-    if (in_topk(i)) part += expf(logits[i] - mx);
+  for_each_logit(logits, n, [&](uint32_t i, float v) {
+    if (in_topk(i, v)) part += expf(v - mx);
+  });
   const float S = block_sum<kSampleThreads>(part, f16s);
   auto prob = [=](float v) { return expf(v - mx) / S; };
   // 3. Top-p: the shortest prefix reaching top_p (all candidates when none does).
   bool reached = false;
-  Cut topp = mass_cut(logits, n, mass_fixed(a.top_p), true, in_topk, prob, bins, u16, sel_s, above_s, &reached);
+  Cut topp = mass_cut_list(logits, n, mass_fixed(a.top_p), true, in_topk, prob, L, bins, u16, sel_s, above_s, &reached);
   if (!reached) topp = topk;
   // 4. Min-p: drop candidates below the first one's probability times min_p.
   const float floor_p = (1.0f / S) * a.min_p;
-  auto kept = [&](uint32_t i) {
-    const float v = logits[i];
-    return in_topk(i) && before_cut(ord_key(v), i, topp) && prob(v) >= floor_p;
+  auto kept = [&](uint32_t i, float v) {
+    return in_topk(i, v) && before_cut(ord_key(v), i, topp) && prob(v) >= floor_p;
   };
   // 5. Temperature over the kept log-probabilities, then the draw.
   const float l0 = logf(1.0f / S);
   const float T = a.temperature;
   auto tq = [=](float v) { return expf((logf(expf(v - mx) / S) - l0) / T); };
   float qp = 0.f;
-  for (uint32_t i = tid; i < n; i += kSampleThreads)
-    if (kept(i)) qp += tq(logits[i]);
+  for_each_logit(logits, n, [&](uint32_t i, float v) {
+    if (kept(i, v)) qp += tq(v);
+  });
   const float Sq = block_sum<kSampleThreads>(qp, f16s);
   __shared__ float draw_s;
   if (tid == 0) draw_s = next_draw(a);
   __syncthreads();
   const float u = draw_s;
   bool got = false;
-  const Cut c = mass_cut(logits, n, mass_fixed(u), false, kept, [=](float v) { return tq(v) / Sq; }, bins, u16, sel_s,
-                         above_s, &got);
+  const Cut c = mass_cut_list(logits, n, mass_fixed(u), false, kept, [=](float v) { return tq(v) / Sq; }, L, bins, u16,
+                              sel_s, above_s, &got);
   if (tid == 0) *token_s = c.id;
   __syncthreads();
 }
 
 __global__ __launch_bounds__(kSampleThreads) void k_sample(SampleArgs a) {
-  __shared__ float cval[kMaxCandidates];
-  __shared__ uint32_t cidx[kMaxCandidates];
+  __shared__ SampleLds L;
+  float *cval = L.cval;
+  uint32_t *cidx = L.cidx;
   __shared__ uint32_t hist[256];
   __shared__ uint32_t u16[16];
   __shared__ float f16s[16];
   __shared__ uint64_t k16[16];
-  __shared__ uint32_t prefix_s, remain_s, keep_s, token_s;
+  __shared__ uint32_t prefix_s, remain_s, keep_s, token_s, cnt_s[2][16];
   __shared__ uint64_t large_bins[256];
   __shared__ uint32_t large_sel[2];
   __shared__ uint64_t large_above;
@@ -298,10 +471,12 @@ __global__ __launch_bounds__(kSampleThreads) void k_sample(SampleArgs a) {
   if (fabsf(a.penalty - 1.0f) > 1.1920929e-7f) {
     const uint32_t n_recent = a.dpos ? p + 1 : a.n_recent;
     const uint32_t start = n_recent > kRepeatLastN ? n_recent - kRepeatLastN : 0;
-    if (tid < n_recent - start) {
-      const uint32_t tok = a.recent[start + tid];
-      bool first = true;
-      for (uint32_t j = start; j < start + tid; j++) first &= a.recent[j] != tok;
+    if (wave == 0) {  // (kRepeatLastN is one wave)
+      const bool mine = lane < n_recent - start;
+      const uint32_t tok = mine ? a.recent[start + lane] : 0xffffffffu;
+      bool first = mine;
+#pragma unroll
+      for (int j = 0; j < 63; j++) first &= !(j < (int)lane && (uint32_t)__builtin_amdgcn_readlane((int)tok, j) == tok);
       if (first && tok < n) {
         const float l = logits[tok];
         logits[tok] = l > 0.f ? l / a.penalty : l * a.penalty;
@@ -313,10 +488,10 @@ __global__ __launch_bounds__(kSampleThreads) void k_sample(SampleArgs a) {
   // 2. Greedy.
   if (a.temperature <= 0.f) {
     uint64_t best = 0;
-    for (uint32_t i = tid; i < n; i += kSampleThreads) {
-      const uint64_t k = ((uint64_t)ord_key(logits[i]) << 32) | (uint64_t)(0xffffffffu - i);
+    for_each_logit(logits, n, [&](uint32_t i, float v) {
+      const uint64_t k = ((uint64_t)ord_key(v) << 32) | (uint64_t)(0xffffffffu - i);
       best = best > k ? best : k;
-    }
+    });
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
       const uint64_t o = ((uint64_t)__shfl_xor((uint32_t)(best >> 32), off, 64) << 32) |
@@ -334,10 +509,43 @@ __global__ __launch_bounds__(kSampleThreads) void k_sample(SampleArgs a) {
     // 3. Candidates: the kc largest logits (radix select of the kc-th).
     const uint32_t k = (a.top_k > 0 && a.top_k < n) ? a.top_k : n;
     if (k > kMaxCandidates) {
-      sample_large(a, k, large_bins, u16, f16s, large_sel, &large_above, &token_s);
+      sample_large(a, k, L, large_bins, u16, f16s, large_sel, &large_above, &token_s);
       goto store;
     }
     const uint32_t kc = k < kMaxCandidates ? k : kMaxCandidates;
+    uint32_t listed = 0;  // entries of the list, at least kc when not 0
+    if (kc <= kFastTopK && kc < n) {
+      // A key that at least kc of the threads' maxima reach, found by
+      // bisection until at most 32 too many do: no logit below it is among
+      // the kc largest, and few above it are not.
+      uint32_t best = 0;
+      for_each_logit(logits, n, [&](uint32_t, float v) { best = max(best, ord_key(v)); });
+      if (tid == 0) L.count = 0;
+      uint32_t lo = 0, hi = 0xffffffffu;  // reached by at least kc; (taken as) reached by fewer
+      for (int it = 0; it < 32 && hi - lo > 1; it++) {
+        const uint32_t mid = lo + (hi - lo) / 2;
+        const uint64_t m = __builtin_amdgcn_ballot_w64(best >= mid);
+        if (lane == 0) cnt_s[it & 1][wave] = (uint32_t)__popcll(m);
+        __syncthreads();
+        uint32_t c = 0;
+#pragma unroll
+        for (int w = 0; w < 16; w++) c += cnt_s[it & 1][w];
+        if (c >= kc) {
+          lo = mid;
+          if (c <= kc + 32) break;
+        } else {
+          hi = mid;
+        }
+      }
+      __syncthreads();
+      for_each_logit(logits, n, [&](uint32_t i, float v) { append(ord_key(v) >= lo, v, i, cval, cidx, &L.count); });
+      __syncthreads();
+      // (More than the list holds: many of the largest logits fell to few
+      // threads.  The radix select below takes those.)
+      listed = L.count <= kMaxCandidates ? L.count : 0;
+      __syncthreads();
+    }
+    if (!listed) {
     uint32_t prefix = 0, need = kc;  // the threshold's key bits so far, and how many of its bucket to take
     if (kc < n) {
       for (int shift = 24; shift >= 0; shift -= 8) {
@@ -401,35 +609,18 @@ __global__ __launch_bounds__(kSampleThreads) void k_sample(SampleArgs a) {
         }
       }
     }
-    uint32_t m = kc;  // candidates, padded to a power of two for the sort
+      listed = kc;
+    }
+    const uint32_t m = kc;  // candidates; the list, padded to a power of two, is sorted
     uint32_t P = 1;
-    while (P < m) P <<= 1;
-    for (uint32_t i = m + tid; i < P; i += kSampleThreads) {
+    while (P < listed) P <<= 1;
+    for (uint32_t i = listed + tid; i < P; i += kSampleThreads) {
       cval[i] = -INFINITY;
       cidx[i] = 0xffffffffu;
     }
     __syncthreads();
-    // 4a. Bitonic sort: logit descending, id ascending on ties.
-    for (uint32_t size = 2; size <= P; size <<= 1) {
-      for (uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
-        for (uint32_t i = tid; i < P; i += kSampleThreads) {
-          const uint32_t j = i ^ stride;
-          if (j > i) {
-            const bool desc = (i & size) == 0;
-            const float vi = cval[i], vj = cval[j];
-            const uint32_t ii = cidx[i], ij = cidx[j];
-            const bool i_first = vi > vj || (vi == vj && ii < ij);
-            if (desc != i_first) {
-              cval[i] = vj;
-              cval[j] = vi;
-              cidx[i] = ij;
-              cidx[j] = ii;
-            }
-          }
-        }
-        __syncthreads();
-      }
-    }
+    // 4a. Sort: logit descending, id ascending on ties.
+    sort_candidates(cval, cidx, P);
     // 4b. Softmax at temperature 1 (sampler.rs:82-83, 116-128).
     const float mx = cval[0];
     float sum_part = 0.f;
