@@ -243,7 +243,7 @@ bool run_gdn_recurrence(hipStream_t s, const GdnArgs &a) {
 // which unrolls the per-token recurrence of qwen35.rs:475-511 exactly (in
 // exact arithmetic).  k_gdn_chunk_prep computes W, U, P, diag(gamma) Q, Kt
 // and gamma_C for every (chunk, head) at once: U and W by forward
-// substitution, one thread per column; the decays as differences of a
+// substitution over blocks of 16 tokens; the decays as differences of a
 // float64 running sum of log-decays.  k_gdn_chunk_scan then carries the
 // state through the chunks: each column of S evolves on its own, so a
 // workgroup owns NC columns of one head and walks the chunks in order.
@@ -262,14 +262,34 @@ __host__ __device__ constexpr uint64_t gdn_chunk_floats(uint32_t kd, uint32_t vd
   return 64ull * (3ull * kd + vd) + 64ull * 64ull + 64ull;
 }
 
+typedef float gdn4_t __attribute__((ext_vector_type(4)));
+
+// Whether no lane of the wave holds an infinity or a NaN.
+__device__ __forceinline__ bool wave_finite(gdn4_t v) {
+  bool bad = false;
+#pragma unroll
+  for (int i = 0; i < 4; i++) bad |= (__float_as_uint(v[i]) & 0x7f800000u) == 0x7f800000u;
+  return __ballot(bad) == 0;
+}
+
+// One workgroup of 8 waves per (chunk, head).  K K^T and Q K^T, the blocks
+// of 16 tokens below the diagonal of the solve and the diagonal blocks'
+// inverses (taken by substitution, 16 x 16) times the right-hand sides all
+// run on f32 MFMAs: element i of an accumulator is row 4·(lane/16) + i, which
+// a B operand reads at k-step i when the A operand takes its columns in that
+// order, so a solved block feeds the next blocks from registers.  512 tokens,
+// 16 heads of 128 x 128: 22 us; with one thread per column of [W | U]
+// and FMA products it took 55, most of it LDS reads.
 template <int KD>
-__global__ __launch_bounds__(256) void k_gdn_chunk_prep(GdnArgs a, float *__restrict__ scratch, uint32_t n_chunks) {
-  constexpr int C = kGdnC, KP = KD + 1, R = KD / 64;
-  __shared__ float qs[C][KP], ks[C][KP];
-  __shared__ __align__(16) float amT[C][C + 4];  // A transposed: amT[u][t] = A[t][u]
-  __shared__ float bs[C], wgam[C];
+__global__ __launch_bounds__(512) void k_gdn_chunk_prep(GdnArgs a, float *__restrict__ scratch, uint32_t n_chunks) {
+  constexpr int C = kGdnC, KP = KD + 4, R = KD / 64, B = C / 16, KB = KD / 16, TP = 20;
+  __shared__ __align__(16) float qs[C][KP], ks[C][KP];
+  __shared__ __align__(16) float am[C][C + 4];    // -A, the blocks on and below the diagonal
+  __shared__ __align__(16) float inv[B][16][TP];  // (I + A)^-1 of each diagonal block
+  __shared__ float bs[C], wgam[C], gq[C], gk[C];
   __shared__ double lg[C];
-  const uint32_t tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
+  const uint32_t tid = threadIdx.x, lane = tid % 64, n = lane % 16, quad = lane / 16;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid / 64);
   const uint32_t chunk = blockIdx.x, head = blockIdx.y;
   const uint32_t vd = a.v_dim;
   const uint32_t t0 = chunk * C, L = min((uint32_t)C, a.n_tokens - t0);
@@ -277,49 +297,52 @@ __global__ __launch_bounds__(256) void k_gdn_chunk_prep(GdnArgs a, float *__rest
   float *base = scratch + ((uint64_t)head * n_chunks + chunk) * gdn_chunk_floats(KD, vd);
   float *Wg = base, *Ug = Wg + C * KD, *Qg = Ug + (uint64_t)C * vd, *Kt = Qg + C * KD, *Pg = Kt + C * KD;
   float *gC = Pg + C * C;
-  // The value column this thread solves first (column tid of [W | U] when it
-  // is a U column), loaded before anything else: nothing before the forward
-  // substitution depends on it.
-  const bool pre_u = tid >= (uint32_t)KD && tid < KD + vd;
-  float vpre[C];
-  {
-    const float *v = a.y + (uint64_t)t0 * conv_dim + 2 * key_dim + head * vd + (pre_u ? tid - KD : 0);
-#pragma unroll
-    for (int t = 0; t < C; t++) vpre[t] = pre_u && (uint32_t)t < L ? v[(uint64_t)t * conv_dim] : 0.f;
-  }
   // The l2-normalised query (times q_scale) and key of each token
   // (qwen35.rs:464-470); rows past the chunk's end are zero.  Wave w takes
-  // tokens w, w+4, ..., all of their loads issued before any is used.
-  {
-    constexpr int TW = C / 4;  // tokens per wave
-    float q[TW][R], k[TW][R];
+  // tokens w, w+8, ..., all of their loads issued before any is used; the
+  // value columns of the wave's first U tile are requested behind them.
+  constexpr int TW = C / 8;  // tokens per wave
+  float q[TW][R], k[TW][R];
 #pragma unroll
-    for (int jj = 0; jj < TW; jj++) {
-      const uint32_t j = wave + 4 * jj;
-      const float *tok = a.y + (uint64_t)(t0 + min(j, L - 1)) * conv_dim;
+  for (int jj = 0; jj < TW; jj++) {
+    const uint32_t j = wave + 8 * jj;
+    const float *tok = a.y + (uint64_t)(t0 + min(j, L - 1)) * conv_dim;
 #pragma unroll
-      for (int i = 0; i < R; i++) {
-        q[jj][i] = j < L ? tok[key_head * KD + lane * R + i] : 0.f;
-        k[jj][i] = j < L ? tok[key_dim + key_head * KD + lane * R + i] : 0.f;
-      }
+    for (int i = 0; i < R; i++) {
+      q[jj][i] = j < L ? tok[key_head * KD + lane * R + i] : 0.f;
+      k[jj][i] = j < L ? tok[key_dim + key_head * KD + lane * R + i] : 0.f;
     }
+  }
+  // Column 16·tile + n of V, rows 16b + 4·quad + i.
+  gdn4_t v[B];
+  auto load_v = [&](uint32_t tile) __attribute__((always_inline)) {
+    const float *col = a.y + (uint64_t)t0 * conv_dim + 2 * key_dim + head * vd + min(16 * tile + n, vd - 1);
 #pragma unroll
-    for (int jj = 0; jj < TW; jj++) {
-      const uint32_t j = wave + 4 * jj;
-      float sq = 0.f, sk = 0.f;
+    for (int b = 0; b < B; b++)
 #pragma unroll
-      for (int i = 0; i < R; i++) {
-        sq = fmaf(q[jj][i], q[jj][i], sq);
-        sk = fmaf(k[jj][i], k[jj][i], sk);
+      for (int i = 0; i < 4; i++) {
+        const uint32_t t = 16 * b + 4 * quad + i;
+        const float x = col[(uint64_t)min(t, L - 1) * conv_dim];
+        v[b][i] = t < L ? x : 0.f;
       }
-      sq = wave_sum(sq);
-      sk = wave_sum(sk);
-      const float fq = a.q_scale / sqrtf(sq + 1e-6f), fk = 1.0f / sqrtf(sk + 1e-6f);
+  };
+  load_v(wave);
 #pragma unroll
-      for (int i = 0; i < R; i++) {
-        qs[j][lane * R + i] = q[jj][i] * fq;
-        ks[j][lane * R + i] = k[jj][i] * fk;
-      }
+  for (int jj = 0; jj < TW; jj++) {
+    const uint32_t j = wave + 8 * jj;
+    float sq = 0.f, sk = 0.f;
+#pragma unroll
+    for (int i = 0; i < R; i++) {
+      sq = fmaf(q[jj][i], q[jj][i], sq);
+      sk = fmaf(k[jj][i], k[jj][i], sk);
+    }
+    sq = wave_sum(sq);
+    sk = wave_sum(sk);
+    const float fq = a.q_scale / sqrtf(sq + 1e-6f), fk = 1.0f / sqrtf(sk + 1e-6f);
+#pragma unroll
+    for (int i = 0; i < R; i++) {
+      qs[j][lane * R + i] = q[jj][i] * fq;
+      ks[j][lane * R + i] = k[jj][i] * fk;
     }
   }
   // Gates: beta, and the running sum of the log-decays in float64.
@@ -332,96 +355,149 @@ __global__ __launch_bounds__(256) void k_gdn_chunk_prep(GdnArgs a, float *__rest
       b = a.raw_gates ? sigmoid_f(rb) : rb;
       l = a.raw_gates ? a.a[head] * softplus_f(rd + a.dt_bias[head]) : logf(rd);
     }
-    double v = l;
+    double s = l;
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
-      const double o = __shfl_up(v, off, 64);
-      if (lane >= (uint32_t)off) v += o;
+      const double o = __shfl_up(s, off, 64);
+      if (lane >= (uint32_t)off) s += o;
     }
+    const double lC = __shfl(s, (int)L - 1, 64);
     bs[lane] = b;
-    lg[lane] = v;
-    wgam[lane] = lane < L ? b * expf((float)v) : 0.f;
+    lg[lane] = s;
+    wgam[lane] = lane < L ? b * expf((float)s) : 0.f;
+    gq[lane] = lane < L ? expf((float)s) : 0.f;
+    gk[lane] = lane < L ? expf((float)(lC - s)) : 0.f;
+    if (lane == 0) gC[0] = expf((float)lC);
   }
   __syncthreads();
-  const double lC = lg[L - 1];
-  // A (strictly lower) and P (lower with the diagonal): 4x4 blocks per thread.
+  // Waves 0-3: A's row block `wave`; waves 4-7: P's, the longest beside the
+  // shortest of A on a SIMD.  Blocks above the diagonal are zero.
   {
-    const uint32_t ti = tid / 16, si = tid % 16;
-    float kk[4][4] = {}, qk[4][4] = {};
-    for (int r = 0; r < KD; r++) {
-      float kt[4], qt[4], kv[4];
+    const bool is_a = wave < 4;
+    const uint32_t rb = is_a ? wave : 7 - wave;
+    const float *rows = is_a ? &ks[16 * rb + n][0] : &qs[16 * rb + n][0];
+    gdn4_t acc[B];
+#pragma unroll
+    for (int b = 0; b < B; b++) acc[b] = gdn4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int kb = 0; kb < KB; kb++) {
+      const gdn4_t rv = *reinterpret_cast<const gdn4_t *>(rows + 16 * kb + 4 * quad);
+#pragma unroll
+      for (int b = 0; b < B; b++) {
+        if ((uint32_t)b > rb) continue;  // (uniform over the wave)
+        const gdn4_t cv = *reinterpret_cast<const gdn4_t *>(&ks[16 * b + n][16 * kb + 4 * quad]);
+#pragma unroll
+        for (int i = 0; i < 4; i++) acc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(rv[i], cv[i], acc[b], 0, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int b = 0; b < B; b++)
 #pragma unroll
       for (int i = 0; i < 4; i++) {
-        kt[i] = ks[4 * ti + i][r];
-        qt[i] = qs[4 * ti + i][r];
-        kv[i] = ks[4 * si + i][r];
-      }
-#pragma unroll
-      for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-          kk[i][j] = fmaf(kt[i], kv[j], kk[i][j]);
-          qk[i][j] = fmaf(qt[i], kv[j], qk[i][j]);
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        const uint32_t t = 4 * ti + i, u = 4 * si + j;
+        const uint32_t t = 16 * rb + 4 * quad + i, u = 16 * b + n;
         const float dec = (u <= t && t < L) ? expf((float)(lg[t] - lg[u])) : 0.f;
-        amT[u][t] = u < t ? bs[t] * dec * kk[i][j] : 0.f;
-        Pg[gdn_frag(t, u, C / 16)] = dec * qk[i][j];
+        // (Selected, not multiplied, to zero: a later token may not be finite.)
+        if (is_a)
+          am[t][u] = u < t ? -(bs[t] * dec * acc[b][i]) : 0.f;
+        else
+          Pg[gdn_frag(t, u, B)] = u <= t ? dec * acc[b][i] : 0.f;
       }
   }
-  // diag(gamma) Q and Kt, and gamma_C.
-  // (The inverse of gdn_frag: Q by (token, r), Kt by (r, token).)
-  for (uint32_t e = tid; e < (uint32_t)(C * KD); e += 256) {
-    const uint32_t l = e / 4 % 64, blk = e / 256, row = l % 16, col = 4 * (e % 4) + l / 16;
-    const uint32_t t = 16 * (blk / (KD / 16)) + row, r = 16 * (blk % (KD / 16)) + col;
-    Qg[e] = t < L ? expf((float)lg[t]) * qs[t][r] : 0.f;
-    const uint32_t r2 = 16 * (blk / (C / 16)) + row, t2 = 16 * (blk % (C / 16)) + col;
-    Kt[e] = t2 < L ? expf((float)(lC - lg[t2])) * ks[t2][r2] : 0.f;
+  // diag(gamma) Q and Kt, by the four floats of a lane of the scan.
+  for (uint32_t e = tid; e < (uint32_t)(C * KD / 4); e += 512) {
+    const uint32_t l = e % 64, blk = e / 64, row = l % 16;
+    const uint32_t t = 16 * (blk / KB) + row, r = 16 * (blk % KB) + l / 16;
+    const uint32_t r2 = 16 * (blk / B) + row, t2 = 16 * (blk % B) + l / 16;
+    gdn4_t qv, kv;
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+      qv[s] = gq[t] * qs[t][r + 4 * s];
+      kv[s] = gk[t2 + 4 * s] * ks[t2 + 4 * s][r2];
+    }
+    *reinterpret_cast<gdn4_t *>(Qg + 4ull * e) = qv;
+    *reinterpret_cast<gdn4_t *>(Kt + 4ull * e) = kv;
   }
-  if (tid == 0) gC[0] = expf((float)lC);
   __syncthreads();
-  // W and U by forward substitution, x_t = rhs_t - sum_{s<t} A[t][s] x_s,
-  // one thread per column of [W | U].
-  for (uint32_t col = tid; col < KD + vd; col += 256) {
-    float x[C];
-    if (col < KD) {
+  // The inverse of diagonal block `wave`, a column per lane of 16.
+  if (wave < B) {
+    float x[16];
 #pragma unroll
-      for (int t = 0; t < C; t++) x[t] = wgam[t] * ks[t][col];
-    } else if (col == tid) {
+    for (int t = 0; t < 16; t++) {
+      x[t] = n == (uint32_t)t ? 1.f : 0.f;
+      float row[16];
 #pragma unroll
-      for (int t = 0; t < C; t++) x[t] = (uint32_t)t < L ? bs[t] * vpre[t] : 0.f;
-    } else {
-      const float *v = a.y + (uint64_t)t0 * conv_dim + 2 * key_dim + head * vd + (col - KD);
+      for (int u4 = 0; u4 < (t + 3) / 4; u4++)
+        *reinterpret_cast<gdn4_t *>(&row[4 * u4]) =
+            *reinterpret_cast<const gdn4_t *>(&am[16 * wave + t][16 * wave + 4 * u4]);
 #pragma unroll
-      for (int t = 0; t < C; t++) x[t] = (uint32_t)t < L ? bs[t] * v[(uint64_t)t * conv_dim] : 0.f;
+      for (int u = 0; u < t; u++) x[t] = fmaf(row[u], x[u], x[t]);
     }
-    // Column by column: once x_u is final it enters every later row, so
-    // each step has up to 63 independent FMAs (a row-by-row loop waits on
-    // one dependent chain of 2016).  Every row still adds its terms in
-    // order u = 0, 1, ..., as the row-by-row form does.
+    if (quad == 0) {
 #pragma unroll
-    for (int u = 0; u < C - 1; u++) {
-      // Rows u+1 .. C-1 of column u, four per 16-byte LDS read.
+      for (int t = 0; t < 16; t++) inv[wave][t][n] = x[t];
+    }
+  }
+  __syncthreads();
+  // X_b = inv_b (rhs_b - sum_{j<b} A_bj X_j), 16 columns of [W | U] at a time.
+  // A block that is not finite is substituted row by row: the inverse's
+  // zeros would carry its infinities and NaNs back to earlier tokens.
+  auto solve = [&](gdn4_t (&x)[B]) __attribute__((always_inline)) {
 #pragma unroll
-      for (int t4 = (u + 1) / 4; t4 < C / 4; t4++) {
-        const float4 a4 = *reinterpret_cast<const float4 *>(&amT[u][4 * t4]);
-        const float av[4] = {a4.x, a4.y, a4.z, a4.w};
+    for (int b = 0; b < B; b++) {
 #pragma unroll
-        for (int i = 0; i < 4; i++)
-          if (4 * t4 + i > u) x[4 * t4 + i] = fmaf(-av[i], x[u], x[4 * t4 + i]);
+      for (int j = 0; j < b; j++) {
+        const gdn4_t av = *reinterpret_cast<const gdn4_t *>(&am[16 * b + n][16 * j + 4 * quad]);
+#pragma unroll
+        for (int i = 0; i < 4; i++) x[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i], x[j][i], x[b], 0, 0, 0);
       }
+      if (!wave_finite(x[b])) {
+#pragma unroll 1
+        for (uint32_t uq = 0; uq < 4; uq++)
+#pragma unroll
+          for (uint32_t ui = 0; ui < 4; ui++) {
+            const float xu = __shfl(x[b][ui], (int)(16 * uq + n), 64);
+#pragma unroll
+            for (uint32_t i = 0; i < 4; i++)
+              if (4 * quad + i > 4 * uq + ui)
+                x[b][i] = fmaf(am[16 * b + 4 * quad + i][16 * b + 4 * uq + ui], xu, x[b][i]);
+          }
+        continue;
+      }
+      const gdn4_t iv = *reinterpret_cast<const gdn4_t *>(&inv[b][n][4 * quad]);
+      gdn4_t y = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < 4; i++) y = __builtin_amdgcn_mfma_f32_16x16x4f32(iv[i], x[b][i], y, 0, 0, 0);
+      x[b] = y;
     }
-    if (col < KD) {
+  };
+  for (uint32_t tile = wave; tile < (uint32_t)KB; tile += 8) {
+    gdn4_t x[B];
 #pragma unroll
-      for (int t = 0; t < C; t++) Wg[gdn_frag(t, col, KD / 16)] = -x[t];  // (the scan adds -W S0)
-    } else {
+    for (int b = 0; b < B; b++)
 #pragma unroll
-      for (int t = 0; t < C; t++) Ug[(uint64_t)t * vd + (col - KD)] = x[t];
+      for (int i = 0; i < 4; i++) {
+        const uint32_t t = 16 * b + 4 * quad + i;
+        x[b][i] = wgam[t] * ks[t][16 * tile + n];
+      }
+    solve(x);
+#pragma unroll
+    for (int b = 0; b < B; b++)
+#pragma unroll
+      for (int i = 0; i < 4; i++)  // (the scan adds -W S0)
+        Wg[gdn_frag(16 * b + 4 * quad + i, 16 * tile + n, KB)] = -x[b][i];
+  }
+  for (uint32_t tile = wave; 16 * tile < vd; tile += 8) {
+    if (tile != wave) load_v(tile);
+#pragma unroll
+    for (int b = 0; b < B; b++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) v[b][i] *= bs[16 * b + 4 * quad + i];
+    solve(v);
+    if (16 * tile + n < vd) {  // (a last tile of 8 columns)
+#pragma unroll
+      for (int b = 0; b < B; b++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) Ug[(uint64_t)(16 * b + 4 * quad + i) * vd + 16 * tile + n] = v[b][i];
     }
   }
 }
@@ -435,14 +511,14 @@ __global__ __launch_bounds__(256) void k_gdn_chunk_prep(GdnArgs a, float *__rest
 // chain of chunks, 112 MFMAs of 32 cycles per wave and chunk (heads of 128):
 // 512 tokens, 16 heads of 128 x 128: 29 us (the FMA form with the matrices
 // staged in LDS took 99).
-typedef float gdn4_t __attribute__((ext_vector_type(4)));
 
 template <int KD>
 __global__ __launch_bounds__(256) void k_gdn_chunk_scan(GdnArgs a, const float *__restrict__ scratch,
                                                         uint32_t n_chunks) {
   constexpr int C = kGdnC, NC = 16, KB = KD / 16, CB = C / 16, MT = KD / 64;
   __shared__ __align__(16) float s_s[KD * NC], d_s[C * NC];
-  const uint32_t tid = threadIdx.x, wave = tid / 64, lane = tid % 64, vd = a.v_dim;
+  const uint32_t tid = threadIdx.x, lane = tid % 64, vd = a.v_dim;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid / 64);
   // Blocks are numbered so that the column blocks of one head run on one
   // XCD (workgroup i goes to XCD i % 8) and share its L2.
   const uint32_t n_cb = (vd + NC - 1) / NC, total = n_cb * a.n_v;
@@ -513,7 +589,12 @@ __global__ __launch_bounds__(256) void k_gdn_chunk_scan(GdnArgs a, const float *
     load_wq(next);
     __builtin_amdgcn_sched_barrier(0);
     lds_barrier();  // D is whole; S0 is spent
-    // O += P D, S_C = gamma_C S0 + Kt^T D.
+    // O += P D, S_C = gamma_C S0 + Kt^T D.  P is zero above its diagonal, and
+    // a later token's infinities and NaNs may not meet those zeros: the wave
+    // leaves out the blocks past its own, and takes its own by selected FMAs
+    // if its deltas are not finite.
+    const bool finite = wave_finite(d);
+    const uint32_t p_blocks = wave + (finite ? 1 : 0);
 #pragma unroll
     for (int m = 0; m < MT; m++)
 #pragma unroll
@@ -523,9 +604,20 @@ __global__ __launch_bounds__(256) void k_gdn_chunk_scan(GdnArgs a, const float *
       const gdn4_t dv = *reinterpret_cast<const gdn4_t *>(&d_s[(b * 64 + lane) * 4]);
 #pragma unroll
       for (int s = 0; s < 4; s++) {
-        o = __builtin_amdgcn_mfma_f32_16x16x4f32(pf[b][s], dv[s], o, 0, 0, 0);
+        if ((uint32_t)b < p_blocks) o = __builtin_amdgcn_mfma_f32_16x16x4f32(pf[b][s], dv[s], o, 0, 0, 0);
 #pragma unroll
         for (int m = 0; m < MT; m++) st[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[m][b][s], dv[s], st[m], 0, 0, 0);
+      }
+    }
+    if (!finite) {
+#pragma unroll 1
+      for (uint32_t t = 0; t < 16; t++) {
+        const float dv = d_s[(wave * 64 + lane % 16 + 16 * (t % 4)) * 4 + t / 4];
+#pragma unroll
+        for (uint32_t i = 0; i < 4; i++) {
+          const float pv = base0[c * per_chunk + p_at + gdn_frag(16 * wave + 4 * quad + i, 16 * wave + t, CB)];
+          o[i] = t <= 4 * quad + i ? fmaf(pv, dv, o[i]) : o[i];
+        }
       }
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -565,10 +657,10 @@ bool run_gdn_chunked(hipStream_t s, const GdnArgs &a, float *scratch) {
   const dim3 prep(n_chunks, a.n_v);
   const uint32_t scan = a.n_v * ((a.v_dim + 15) / 16);
   if (a.k_dim == 64) {
-    k_gdn_chunk_prep<64><<<prep, 256, 0, s>>>(a, scratch, n_chunks);
+    k_gdn_chunk_prep<64><<<prep, 512, 0, s>>>(a, scratch, n_chunks);
     k_gdn_chunk_scan<64><<<scan, 256, 0, s>>>(a, scratch, n_chunks);
   } else {
-    k_gdn_chunk_prep<128><<<prep, 256, 0, s>>>(a, scratch, n_chunks);
+    k_gdn_chunk_prep<128><<<prep, 512, 0, s>>>(a, scratch, n_chunks);
     k_gdn_chunk_scan<128><<<scan, 256, 0, s>>>(a, scratch, n_chunks);
   }
   return true;
