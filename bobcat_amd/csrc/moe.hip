@@ -424,10 +424,12 @@ bool run_experts_down(hipStream_t s, uint32_t format, const uint8_t *W, uint32_t
 // workgroup of 16 waves; wave w takes a contiguous run of the entries.  The
 // entries' experts are first copied to LDS as bytes (up to
 // kGroupLdsEntries entries; larger batches read them from the route).  Each
-// wave counts its run's entries per expert 64 at a time, one ballot per
-// distinct expert among the 64; a prefix over (expert, wave) gives every
-// wave its first slot for each expert; a second pass over the run places
-// the entries, so each expert's entries keep their order.
+// wave counts its run's entries per expert 64 at a time, one ballot per bit
+// of the expert id finding the lanes of the same expert, the lowest of which
+// counts for all; a prefix over (expert, wave) gives every wave its first
+// slot for each expert; a second pass over the run places the entries, so
+// each expert's entries keep their order.  Bound by latency: 2,048 entries
+// of 32 experts in 5 us (22 with one turn per distinct expert of the 64).
 constexpr int kGroupWaves = 16;
 constexpr uint32_t kGroupLdsEntries = 16384;
 static_assert(kMoeMaxExperts <= 256, "expert ids fit a byte");
@@ -450,48 +452,56 @@ __global__ __launch_bounds__(kGroupWaves * 64) void k_moe_group(const uint32_t *
   const uint32_t per = (n_entries + kGroupWaves * 64 - 1) / (kGroupWaves * 64) * 64;  // entries per wave
   const uint32_t v0 = min(wave * per, n_entries), v1 = min(v0 + per, n_entries);
   const uint64_t below = (1ull << lane) - 1;
-  // For each distinct expert le among this slice's lanes (those with v < v1),
-  // in order of the lowest lane holding it: fn(le, ballot of its lanes).
-  auto distinct = [&](uint32_t e, bool valid, auto fn) {
-    uint64_t todo = __ballot(valid);
-    while (todo) {
-      const uint32_t leader = (uint32_t)__ffsll((unsigned long long)todo) - 1;
-      const uint32_t le = __shfl(e, leader, 64);
-      const uint64_t mask = __ballot(valid && e == le);
-      fn(le, mask);
-      todo &= ~mask;
+  // The lanes of this slice (those valid) whose expert is this lane's.
+  const uint32_t bits = 32 - __clz((int)(n_experts - 1));  // (n_experts 1: 0)
+  auto peers = [&](uint32_t e, bool valid) {
+    uint64_t mask = __ballot(valid);
+    for (uint32_t b = 0; b < bits; b++) {
+      const uint64_t set = __ballot(e >> b & 1);
+      mask &= e >> b & 1 ? set : ~set;
     }
+    return mask;
   };
   for (uint32_t first = v0; first < v1; first += 64) {
     const uint32_t v = first + lane;
     const bool valid = v < v1;
     const uint32_t e = valid ? expert_of(v) : 0;
-    distinct(e, valid, [&](uint32_t le, uint64_t mask) {
-      if (lane == 0) slot[wave][le] += (uint32_t)__popcll(mask);
-    });
+    const uint64_t mask = peers(e, valid);
+    if (valid && (mask & below) == 0) slot[wave][e] += (uint32_t)__popcll(mask);
+    __builtin_amdgcn_wave_barrier();
   }
   __syncthreads();
-  // Expert totals, their exclusive prefix (offsets), then each wave's first
-  // slot per expert.
+  // Expert totals, their exclusive prefix (offsets; wave 0, by shuffles),
+  // then each wave's first slot per expert.
   for (uint32_t e = threadIdx.x; e < n_experts; e += kGroupWaves * 64) {
     uint32_t t = 0;
+#pragma unroll
     for (int w = 0; w < kGroupWaves; w++) t += slot[w][e];
     total[e] = t;
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
+  if (wave == 0) {
     uint32_t start = 0;
-    for (uint32_t e = 0; e < n_experts; e++) {
-      const uint32_t t = total[e];
-      total[e] = start;
-      offsets[e] = start;
-      start += t;
+    for (uint32_t e0 = 0; e0 < n_experts; e0 += 64) {
+      const uint32_t e = e0 + lane, t = e < n_experts ? total[e] : 0;
+      uint32_t upto = t;
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t o = __shfl_up(upto, off, 64);
+        if (lane >= (uint32_t)off) upto += o;
+      }
+      if (e < n_experts) {
+        total[e] = start + upto - t;
+        offsets[e] = start + upto - t;
+      }
+      start += __shfl(upto, 63, 64);
     }
-    offsets[n_experts] = start;
+    if (lane == 0) offsets[n_experts] = start;
   }
   __syncthreads();
   for (uint32_t e = threadIdx.x; e < n_experts; e += kGroupWaves * 64) {
     uint32_t start = total[e];
+#pragma unroll
     for (int w = 0; w < kGroupWaves; w++) {
       const uint32_t c = slot[w][e];
       slot[w][e] = start;
@@ -503,13 +513,12 @@ __global__ __launch_bounds__(kGroupWaves * 64) void k_moe_group(const uint32_t *
     const uint32_t v = first + lane;
     const bool valid = v < v1;
     const uint32_t e = valid ? expert_of(v) : 0;
-    distinct(e, valid, [&](uint32_t le, uint64_t mask) {
-      const uint32_t base = slot[wave][le];
-      if (valid && e == le) entries[base + (uint32_t)__popcll(mask & below)] = v;
-      __builtin_amdgcn_wave_barrier();
-      if (lane == 0) slot[wave][le] = base + (uint32_t)__popcll(mask);
-      __builtin_amdgcn_wave_barrier();
-    });
+    const uint64_t mask = peers(e, valid);
+    const uint32_t at = slot[wave][e] + (uint32_t)__popcll(mask & below);
+    if (valid) entries[at] = v;
+    __builtin_amdgcn_wave_barrier();
+    if (valid && (mask & below) == 0) slot[wave][e] = at + (uint32_t)__popcll(mask);
+    __builtin_amdgcn_wave_barrier();
   }
 }
 

@@ -1,5 +1,5 @@
 """The chunked DeltaNet form on its tile edges and on values that are not
-finite, against the sequential rule in float64."""
+finite, against the sequential rule in float64; the grouping of expert entries."""
 from __future__ import annotations
 
 import ctypes as C
@@ -59,3 +59,21 @@ def test_chunked_rule_on_edges_and_nonfinite_tokens(hip, n_k, n_v, dk, dv, n_tok
         assert (np.isfinite(g) == finite).all()
         if finite.any():
             assert np.abs(g - w)[finite].max() < 1e-5 * np.abs(w[finite]).max()
+
+
+@pytest.mark.parametrize("n_experts,n_used,n_tokens", [(1, 1, 70), (3, 2, 1), (64, 4, 300), (65, 3, 341), (128, 8, 2049)])
+def test_group_entries_by_expert(hip, n_experts, n_used, n_tokens):
+    """Entries by expert, in token order within: runs of fewer and more than
+    64 entries per wave, ids of 0 to 7 bits, one and two waves' width of
+    experts, ids read from LDS and (above 16,384 entries) from the route."""
+    rng = np.random.default_rng(n_experts)
+    ids = np.stack([rng.choice(n_experts, n_used, replace=False) for _ in range(n_tokens)]).astype(np.uint32)
+    route = hip.buffer_from(np.concatenate([ids, np.zeros_like(ids)], axis=1).reshape(-1))
+    offsets, entries = hip.new_buffer((n_experts + 1) * 4), hip.new_buffer(ids.size * 4)
+    hip.begin()
+    hip.moe_group(route.at(0), offsets.at(0), entries.at(0), n_experts, n_used, n_tokens)
+    hip.end()
+    flat = ids.reshape(-1)
+    assert (hip.read(entries.at(0), np.empty(ids.size, np.uint32)) == np.argsort(flat, kind="stable")).all()
+    counts = np.bincount(flat, minlength=n_experts)
+    assert (hip.read(offsets.at(0), np.empty(n_experts + 1, np.uint32)) == np.concatenate([[0], np.cumsum(counts)])).all()
