@@ -29,6 +29,7 @@
 // wave and block, most of them the softmax and the splitting of p.
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "device.h"
 #include "kernels.h"
@@ -218,18 +219,31 @@ __global__ __launch_bounds__(256, HD == 64 ? 3 : HD == 128 ? 2 : 1) void k_attn_
     l_run += psum;
     // O^T += V^T·P^T over 2 k-steps of 16 keys: lane supplies V^T[32b + col]
     // of keys 16j + 4·half + {0..3, 8..11} and the probabilities of the same.
+    // Keys past the wave's last query may be those of the workgroup's later
+    // queries: their values are left out, as they may not be finite.
+    auto add = [&](auto past) __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < 2; j++) {
+      for (int j = 0; j < 2; j++) {
 #pragma unroll
-      for (int b = 0; b < OB; b++) {
-        const uint32_t d = 32 * b + col;
-        const ph4_t v0 = *reinterpret_cast<const ph4_t *>(&v_s[buf][((4 * j + half_id) * HD + d) * 4]);
-        const ph4_t v1 = *reinterpret_cast<const ph4_t *>(&v_s[buf][((4 * j + 2 + half_id) * HD + d) * 4]);
-        const ph8_t a = __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
-        o[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, ph[j], o[b], 0, 0, 0);
-        o[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, pl[j], o[b], 0, 0, 0);
+        for (int b = 0; b < OB; b++) {
+          const uint32_t d = 32 * b + col;
+          const ph4_t v0 = *reinterpret_cast<const ph4_t *>(&v_s[buf][((4 * j + half_id) * HD + d) * 4]);
+          const ph4_t v1 = *reinterpret_cast<const ph4_t *>(&v_s[buf][((4 * j + 2 + half_id) * HD + d) * 4]);
+          ph8_t a = __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
+          if constexpr (past) {
+#pragma unroll
+            for (int i = 0; i < 8; i++)
+              if (kb + 16 * j + 4 * half_id + (i & 4) * 2 + (i & 3) >= kend) a[i] = (_Float16)0.f;
+          }
+          o[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, ph[j], o[b], 0, 0, 0);
+          o[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, pl[j], o[b], 0, 0, 0);
+        }
       }
-    }
+    };
+    if (kb + kPrefKeys > kend)
+      add(std::true_type{});
+    else
+      add(std::false_type{});
   };
   if (b_lo < b_hi) {
     stage(0);
