@@ -323,7 +323,7 @@ uint64_t attn_prefill_partial_floats(uint32_t n_queries, uint32_t n_heads, uint3
 
 uint32_t attn_prefill_splits(uint32_t n_heads, uint32_t n_kv, uint32_t head_dim, uint32_t first_pos,
                              uint32_t n_queries, uint64_t partial_floats) {
-  if (!n_queries) return 1;
+  if (!n_queries || !n_heads) return 1;
   // Enough workgroups for two per CU (three, which heads of 64 have registers
   // for, made their kernel 4% faster and its combine as much slower), at least kMinSplitBlocks 32-key blocks
   // per split of the batch's middle tile, and no more partials than the
@@ -345,7 +345,7 @@ void run_attn_prefill_mfma(hipStream_t s, const float *q, const void *k_cache, c
                            uint32_t n_queries, uint32_t q_stride, uint32_t out_stride, float scale, float *partials,
                            uint64_t partial_floats, const float *gate, uint32_t gate_head_stride,
                            uint32_t gate_query_stride) {
-  if (!n_queries) return;
+  if (!n_queries || !n_heads) return;
   const uint32_t n_split =
       partials ? attn_prefill_splits(n_heads, n_kv, head_dim, first_pos, n_queries, partial_floats) : 1;
   const uint32_t per_wg = kPrefQ * attn_prefill_tiles(n_heads / n_kv);

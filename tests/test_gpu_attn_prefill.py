@@ -90,3 +90,13 @@ def test_attention_prefill_limits(hip):
             hip.attention_prefill(b.at(0), b.at(0), b.at(0), b.at(0), heads, kv_heads, dim, 0, 1, 16)
         hip.discard()
         assert e.value.status == ATTENTION_LIMITS
+
+
+def test_attention_prefill_without_heads_writes_nothing(hip):
+    """No query heads leave nothing to compute: the call is accepted, as
+    attention accepts it, and the outputs keep their bytes."""
+    before = np.arange(1024, dtype=np.float32)
+    b, out = hip.new_buffer(1 << 20), hip.buffer_from(before)
+    for queries in (0, 1, 70):
+        run(hip, lambda: hip.attention_prefill(b.at(0), b.at(0), b.at(0), out.at(0), 0, 2, 64, 3, queries, 128))
+        assert np.array_equal(hip.read(out.at(0), np.empty(1024, np.float32)), before)
