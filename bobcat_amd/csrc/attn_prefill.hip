@@ -96,7 +96,8 @@ __global__ __launch_bounds__(256, HD == 64 ? 3 : HD == 128 ? 2 : 1) void k_attn_
 
   // The block's cache rows through a descriptor of the block: rows past the
   // end read zeros (their scores are masked), and an address is one constant
-  // per thread.
+  // per thread.  The whole address is in the vector offset: that is what is
+  // compared with the descriptor's size (a scalar offset is not).
   const uint32_t row_bytes = n_kv * HD * 2;
   u32x4_t kr[NP];
   uint32_t vr[NP][4];
@@ -115,7 +116,7 @@ __global__ __launch_bounds__(256, HD == 64 ? 3 : HD == 128 ? 2 : 1) void k_attn_
       const uint32_t c = tid + 256 * p, dp = c % (HD / 2), kq = c / (HD / 2);
 #pragma unroll
       for (int i = 0; i < 4; i++)
-        vr[p][i] = __builtin_amdgcn_raw_buffer_load_b32(vd, 4 * kq * row_bytes + 4 * dp, i * row_bytes, 0);
+        vr[p][i] = __builtin_amdgcn_raw_buffer_load_b32(vd, (4 * kq + i) * row_bytes + 4 * dp, 0, 0);
     }
   };
   auto stage = [&](int buf) __attribute__((always_inline)) {
