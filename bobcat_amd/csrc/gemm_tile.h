@@ -33,6 +33,7 @@
 #include <type_traits>
 #include <utility>
 
+#include "../../include/bobcat_hip.h"
 #include "formats.h"
 #include "frag.h"
 #include "kernels.h"
@@ -451,8 +452,10 @@ __global__ __launch_bounds__(256, 1) void k_gemm(const uint8_t *__restrict__ W, 
   const uint8_t *wrow = PAIR && ar >= OR ? W2 + (uint64_t)min(row0 + ar - OR, n_rows - 1) * row_bytes
                                          : W + (uint64_t)min(row0 + ar, n_rows - 1) * row_bytes;
   // MFMA role: token blocks NB·wt + j of the tile, read through a descriptor
-  // of the lane's block(s) that ends with them: stages past the columns (of
-  // a last super-block that is not whole) read zeros.
+  // of the lane's block(s).  TAIL: formats whose rows need not be whole
+  // super-blocks; the descriptor ends with the columns, and the stages past
+  // them read zeros (load_x).
+  constexpr bool TAIL = !GROUPED && (FMT == BCH_F32 || FMT == BCH_F16 || FMT == BCH_Q8_0 || FMT == BCH_Q4_0);
   __amdgpu_buffer_rsrc_t xr[NB];
   uint32_t xv[NB], xs[NB];
 #pragma unroll
@@ -530,7 +533,11 @@ __global__ __launch_bounds__(256, 1) void k_gemm(const uint8_t *__restrict__ W, 
   const uint32_t last_stage = 4 * sb1 - 1, last_sb = sb1 - 1;
   auto load_x = [&](uint32_t stage, int slot, auto sj) __attribute__((always_inline)) {
     constexpr int s = decltype(sj)::value / NB, j = decltype(sj)::value % NB;
-    x[slot][s][j] = __builtin_amdgcn_raw_buffer_load_b128(xr[j], xv[j], (4 * stage + s) * xs[j], 0);
+    const uint32_t step = (4 * stage + s) * xs[j];
+    if constexpr (TAIL)  // (only the vector offset is sure to be checked against the descriptor's size)
+      x[slot][s][j] = __builtin_amdgcn_raw_buffer_load_b128(xr[j], xv[j] + step, 0, 0);
+    else  // always inside the columns
+      x[slot][s][j] = __builtin_amdgcn_raw_buffer_load_b128(xr[j], xv[j], step, 0);
   };
   auto load_w = [&](auto stage, uint32_t sb) __attribute__((always_inline)) {
     constexpr int S = decltype(stage)::value;

@@ -34,3 +34,14 @@ def test_attention_loads_have_no_scalar_offset(name):
     assert loads
     for _, args in loads:
         assert len(args) == 4 and args[2] == "0", args
+
+
+def test_gemm_loads_past_the_columns_have_no_scalar_offset():
+    """The GEMM's stages past the columns exist for the formats whose rows need
+    not be whole super-blocks of 256 columns: those take the checked form."""
+    text = (CSRC / "gemm_tile.h").read_text()
+    tail = re.search(r"constexpr bool TAIL = !GROUPED && \((.*?)\);", text).group(1)
+    assert set(re.findall(r"BCH_\w+", tail)) == {"BCH_F32", "BCH_F16", "BCH_Q8_0", "BCH_Q4_0"}
+    checked, plain = buffer_loads(text)
+    assert re.search(r"if constexpr \(TAIL\)[^;]*$", text[:checked[0]]) and checked[1][2] == "0"
+    assert re.search(r"else[^;]*$", text[checked[0]:plain[0]])
