@@ -43,6 +43,21 @@ constexpr uint32_t kRepeatLastN = 64;  // REPEAT_LAST_N (sampler.rs:8-9)
 // maxima at or above it, ~-1024·ln(1 - k/1024) logits are (1,420 for 768).
 constexpr uint32_t kFastTopK = 768;
 
+// bins[bin] += w for the lanes with `take`.  Those that share the first such
+// lane's `id` (equal ids: equal bins and weights) add once: masked or equal
+// logits would otherwise queue up on one counter (151,936 logits, all but 10
+// masked, top-k 40: 725 us with one add per lane, 301 so).
+template <class T>
+__device__ __forceinline__ void add_bin(T *bins, uint32_t bin, T w, uint32_t id, bool take) {
+  const uint64_t all = __builtin_amdgcn_ballot_w64(take);
+  if (!all) return;
+  const uint32_t lane = threadIdx.x % 64, lead = (uint32_t)__ffsll((unsigned long long)all) - 1;
+  const bool same = take && id == (uint32_t)__builtin_amdgcn_readlane((int)id, (int)lead);
+  const uint64_t m = __builtin_amdgcn_ballot_w64(same);
+  if (lane == lead) w *= (T)__popcll(m);
+  if (take && (!same || lane == lead)) atomicAdd(&bins[bin], w);
+}
+
 // f(i, logits[i]) for the elements of this thread (i = tid, tid + 1024, ...),
 // eight loads in flight.
 template <class F>
@@ -95,7 +110,7 @@ __device__ __forceinline__ float next_draw(const SampleArgs &a) {
 // Exclusive prefix sum of one value per thread over the workgroup; `total`
 // receives the sum.  Uses shuffles within a wave and LDS across waves.
 template <class T>
-__device__ T block_scan(T v, T *lds16, T *total) {
+__device__ __forceinline__ T block_scan(T v, T *lds16, T *total) {
   const uint32_t lane = threadIdx.x % 64, wave = threadIdx.x / 64;
   T incl = v;
 #pragma unroll
@@ -133,19 +148,19 @@ __device__ __forceinline__ bool before_cut(uint32_t key, uint32_t id, Cut c) {
 // that pass `pred`; 0xffffffff when there are fewer.  Each thread scans a
 // contiguous range, so the order is the id order.
 template <class Pred>
-__device__ uint32_t nth_tied_id(const float *logits, uint32_t n, uint32_t K, uint32_t j, Pred pred, uint32_t *u16,
+__device__ __forceinline__ uint32_t nth_tied_id(const float *logits, uint32_t n, uint32_t K, uint32_t j, Pred pred, uint32_t *u16,
                                 uint32_t *result) {
   const uint32_t per = (n + kSampleThreads - 1) / kSampleThreads;
   const uint32_t lo = threadIdx.x * per, hi = min(n, lo + per);
   uint32_t cnt = 0;
-  for (uint32_t i = lo; i < hi; i++) cnt += ord_key(logits[i]) == K && pred(i);
+  for (uint32_t i = lo; i < hi; i++) cnt += ord_key(logits[i]) == K && pred(i, logits[i]);
   if (threadIdx.x == 0) *result = 0xffffffffu;
   uint32_t total;
   const uint32_t base = block_scan<uint32_t>(cnt, u16, &total);
   if (j >= base && j < base + cnt) {
     uint32_t seen = base;
     for (uint32_t i = lo; i < hi; i++)
-      if (ord_key(logits[i]) == K && pred(i)) {
+      if (ord_key(logits[i]) == K && pred(i, logits[i])) {
         if (seen == j) {
           *result = i;
           break;
@@ -181,7 +196,7 @@ __device__ __forceinline__ uint64_t mass_fixed(float w) { return __double2ull_rn
 // histograms; the elements tied at the final key weigh the same, so the id
 // of the crossing one follows by division.
 template <class Pred, class Weight>
-__device__ Cut mass_cut(const float *logits, uint32_t n, uint64_t target, bool inclusive, Pred pred, Weight weight,
+__device__ __forceinline__ Cut mass_cut(const float *logits, uint32_t n, uint64_t target, bool inclusive, Pred pred, Weight weight,
                         uint64_t *bins, uint32_t *u16, uint32_t *sel_s, uint64_t *above_s, bool *found) {
   constexpr uint32_t kNone = 0xffffffffu;
   const uint32_t tid = threadIdx.x;
@@ -192,36 +207,40 @@ __device__ Cut mass_cut(const float *logits, uint32_t n, uint64_t target, bool i
     for (uint32_t i = tid; i < 256; i += kSampleThreads) bins[i] = 0;
     __syncthreads();
     const uint32_t hi_mask = shift == 24 ? 0u : ~0u << (shift + 8);
-    for (uint32_t i = tid; i < n; i += kSampleThreads) {
-      const float v = logits[i];
+    for_each_logit(logits, n, [&](uint32_t i, float v) {
       const uint32_t key = ord_key(v);
-      if ((key & hi_mask) == (prefix & hi_mask) && pred(i))
-        atomicAdd(reinterpret_cast<unsigned long long *>(&bins[(key >> shift) & 255u]),
-                  (unsigned long long)mass_fixed(weight(v)));
-    }
+      const bool take = (key & hi_mask) == (prefix & hi_mask) && pred(i, v);
+      add_bin(reinterpret_cast<unsigned long long *>(bins), (key >> shift) & 255u,
+              take ? (unsigned long long)mass_fixed(weight(v)) : 0ull, key, take);
+    });
     __syncthreads();
-    if (tid == 0) {
-      uint64_t acc = above;
-      uint32_t bin = kNone, last = kNone;
-      for (int b = 255; b >= 0; b--) {
-        if (bins[b] == 0) continue;
-        const uint64_t next = acc + bins[b];
-        if (inclusive ? next >= target : next > target) {
-          bin = (uint32_t)b;
-          break;
-        }
-        acc = next;
-        last = (uint32_t)b;
+    if (tid < 64) {
+      // Lane l holds bins 255 - 4l .. 252 - 4l, the highest first.
+      uint64_t w[4], upto = 0;
+#pragma unroll
+      for (uint32_t k = 0; k < 4; k++) upto += w[k] = bins[255 - 4 * tid - k];
+      uint64_t acc = above - upto;
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) {
+        const uint64_t o = __shfl_up(upto, off, 64);
+        if (tid >= (uint32_t)off) upto += o;
       }
-      if (bin == kNone) {
-        // Not reached: descend into the last bin with weight, if any.
-        sel_s[0] = last;
-        sel_s[1] = 0;
-        *above_s = last == kNone ? acc : acc - bins[last];
-      } else {
-        sel_s[0] = bin;
-        sel_s[1] = 1;
-        *above_s = acc;
+      acc += upto;
+      uint32_t bin = kNone, last = kNone;
+      uint64_t bin_acc = 0, last_acc = 0;
+#pragma unroll
+      for (uint32_t k = 0; k < 4; k++) {
+        const uint64_t next = acc + w[k];
+        if (w[k] && bin == kNone && (inclusive ? next >= target : next > target)) bin = 255 - 4 * tid - k, bin_acc = acc;
+        if (w[k]) last = 255 - 4 * tid - k, last_acc = acc;
+        acc = next;
+      }
+      const uint64_t hit = __ballot(bin != kNone), any = __ballot(last != kNone);
+      if (tid == (hit ? (uint32_t)__ffsll((unsigned long long)hit) - 1 : 63 - (uint32_t)__clzll((long long)(any | 1)))) {
+        // (Not reached: descend into the last bin with weight, if any.)
+        sel_s[0] = hit ? bin : last;
+        sel_s[1] = hit != 0;
+        *above_s = hit ? bin_acc : last_acc;
       }
     }
     __syncthreads();
@@ -236,7 +255,7 @@ __device__ Cut mass_cut(const float *logits, uint32_t n, uint64_t target, bool i
     prefix |= bin << shift;
   }
   uint32_t c = 0;
-  for (uint32_t i = tid; i < n; i += kSampleThreads) c += ord_key(logits[i]) == prefix && pred(i);
+  for_each_logit(logits, n, [&](uint32_t i, float v) { c += ord_key(v) == prefix && pred(i, v); });
   uint32_t n_tied;
   block_scan<uint32_t>(c, u16, &n_tied);
   uint32_t j = n_tied - 1;
@@ -256,7 +275,7 @@ __device__ Cut mass_cut(const float *logits, uint32_t n, uint64_t target, bool i
 
 // The candidates of a list in LDS, in rank order: logit descending, id
 // ascending.  P (a power of two) entries, the unused ones (-inf, 0xffffffff).
-__device__ void sort_candidates(float *cval, uint32_t *cidx, uint32_t P) {
+__device__ __forceinline__ void sort_candidates(float *cval, uint32_t *cidx, uint32_t P) {
   for (uint32_t size = 2; size <= P; size <<= 1) {
     for (uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
       for (uint32_t i = threadIdx.x; i < P; i += kSampleThreads) {
@@ -312,7 +331,7 @@ struct SampleLds {
 // weights are the same integers, so the cut is mass_cut's; more elements in
 // the bin than the list holds go to mass_cut.
 template <class Pred, class Weight>
-__device__ Cut mass_cut_list(const float *logits, uint32_t n, uint64_t target, bool inclusive, Pred pred, Weight weight,
+__device__ __forceinline__ Cut mass_cut_list(const float *logits, uint32_t n, uint64_t target, bool inclusive, Pred pred, Weight weight,
                              SampleLds &L, uint64_t *bins, uint32_t *u16, uint32_t *sel_s, uint64_t *above_s,
                              bool *found) {
   constexpr uint32_t kPer = kMassBins / kSampleThreads, kNone = 0xffffffffu;
@@ -357,8 +376,7 @@ __device__ Cut mass_cut_list(const float *logits, uint32_t n, uint64_t target, b
   const uint32_t m = L.count;
   if (m > kMaxCandidates) {
     __syncthreads();
-    return mass_cut(logits, n, target, inclusive, [&](uint32_t i) { return pred(i, logits[i]); }, weight, bins, u16, sel_s,
-                    above_s, found);
+    return mass_cut(logits, n, target, inclusive, pred, weight, bins, u16, sel_s, above_s, found);
   }
   uint32_t P = 1;
   while (P < m) P <<= 1;
@@ -396,7 +414,7 @@ __device__ Cut mass_cut_list(const float *logits, uint32_t n, uint64_t target, b
   return c;
 }
 
-__device__ void sample_large(const SampleArgs &a, uint32_t k, SampleLds &L, uint64_t *bins, uint32_t *u16, float *f16s,
+__device__ __forceinline__ void sample_large(const SampleArgs &a, uint32_t k, SampleLds &L, uint64_t *bins, uint32_t *u16, float *f16s,
                              uint32_t *sel_s, uint64_t *above_s, uint32_t *token_s) {
   const uint32_t tid = threadIdx.x, n = a.n;
   const float *logits = a.logits;
@@ -541,7 +559,8 @@ __global__ __launch_bounds__(kSampleThreads) void k_sample(SampleArgs a) {
       for_each_logit(logits, n, [&](uint32_t i, float v) { append(ord_key(v) >= lo, v, i, cval, cidx, &L.count); });
       __syncthreads();
       // (More than the list holds: many of the largest logits fell to few
-      // threads.  The radix select below takes those.)
+      // threads, or are equal, as those of a masked vocabulary.  The radix
+      // select below takes those.)
       listed = L.count <= kMaxCandidates ? L.count : 0;
       __syncthreads();
     }
@@ -552,22 +571,32 @@ __global__ __launch_bounds__(kSampleThreads) void k_sample(SampleArgs a) {
         for (uint32_t i = tid; i < 256; i += kSampleThreads) hist[i] = 0;
         __syncthreads();
         const uint32_t hi_mask = shift == 24 ? 0u : ~0u << (shift + 8);
-        for (uint32_t i = tid; i < n; i += kSampleThreads) {
-          const uint32_t key = ord_key(logits[i]);
-          if ((key & hi_mask) == (prefix & hi_mask)) atomicAdd(&hist[(key >> shift) & 255u], 1u);
-        }
+        for_each_logit(logits, n, [&](uint32_t, float v) {
+          const uint32_t key = ord_key(v), bin = (key >> shift) & 255u;
+          add_bin(hist, bin, 1u, bin, (key & hi_mask) == (prefix & hi_mask));
+        });
         __syncthreads();
-        if (tid == 0) {
-          uint32_t acc = 0, bin = 255;
-          for (int b = 255; b >= 0; b--) {
-            if (acc + hist[b] >= need) {
-              bin = (uint32_t)b;
-              break;
-            }
-            acc += hist[b];
+        if (wave == 0) {
+          // Lane l holds bins 255 - 4l .. 252 - 4l, the highest first; one
+          // bin of all brings the count to `need`.
+          uint32_t h[4], upto = 0;
+#pragma unroll
+          for (uint32_t b = 0; b < 4; b++) upto += h[b] = hist[255 - 4 * lane - b];
+          uint32_t acc = 0u - upto;
+#pragma unroll
+          for (int off = 1; off < 64; off <<= 1) {
+            const uint32_t o = __shfl_up(upto, off, 64);
+            if (lane >= (uint32_t)off) upto += o;
           }
-          prefix_s = prefix | (bin << shift);
-          remain_s = need - acc;
+          acc += upto;
+#pragma unroll
+          for (uint32_t b = 0; b < 4; b++) {
+            if (acc < need && acc + h[b] >= need) {
+              prefix_s = prefix | ((255 - 4 * lane - b) << shift);
+              remain_s = need - acc;
+            }
+            acc += h[b];
+          }
         }
         __syncthreads();
         prefix = prefix_s;

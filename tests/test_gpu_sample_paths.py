@@ -1,8 +1,10 @@
 """The sampler's candidate searches at the sizes and distributions where they
 can go wrong: k around the 768 up to which a bound of the threads' maxima is
 used, fewer logits than threads, ties everywhere, the largest logits all with
-one thread (more listed than the list holds: the radix select), and cuts whose
-bin holds more than the list (top_k = 0 on equal logits).
+one thread (a list of little more than k) or with fewer threads than k (more
+than the list holds: the radix select), most of them masked or all equal (the
+radix select again, whole waves in one bin), and cuts whose bin holds more than
+the list (top_k = 0 on equal logits).
 
 The oracle ranks by logit, then id, as the GPU does, and both take the draw
 `u`: kept away from candidate boundaries (draws of a uniform grid's
@@ -35,11 +37,18 @@ def logits_of(kind, n, rng):
         x = rng.standard_normal(n).astype(np.float32) * 0.1
         x[5::1024] += 8
         return x
+    if kind == "few_threads":  # those of 70 threads, at 65,536 logits 4,480 of them
+        x = rng.standard_normal(n).astype(np.float32) * 0.1
+        x[np.arange(n) % 1024 < 70] += 8
+        return x
+    if kind == "equal":
+        return np.full(n, 2.5, np.float32)
     return np.where(np.arange(n) % 7 == 0, np.float32(0), -np.inf).astype(np.float32)  # "masked"
 
 
-@pytest.mark.parametrize("kind", ["normal", "ties", "one_thread", "masked"])
-@pytest.mark.parametrize("n,top_k", [(100, 20), (1000, 999), (5000, 768), (5000, 769), (65536, 40), (65536, 4000)])
+@pytest.mark.parametrize("kind", ["normal", "ties", "one_thread", "few_threads", "masked", "equal"])
+@pytest.mark.parametrize("n,top_k", [(100, 20), (1000, 999), (5000, 768), (5000, 769), (65536, 40), (65536, 768),
+                                     (65536, 4000)])
 def test_top_k_set(hip, kind, n, top_k):
     """With equal weights for all candidates (a huge temperature) the token
     drawn at u = (i + 0.5) / k is the candidate of rank i."""
@@ -52,7 +61,8 @@ def test_top_k_set(hip, kind, n, top_k):
         assert draw(hip, x, st, (i + 0.5) / len(order)) == order[i], i
 
 
-@pytest.mark.parametrize("kind,n", [("normal", 65536), ("normal", 300), ("ties", 30000), ("one_thread", 20000)])
+@pytest.mark.parametrize("kind,n", [("normal", 65536), ("normal", 300), ("ties", 30000), ("one_thread", 20000),
+                                    ("equal", 30001)])
 @pytest.mark.parametrize("top_k,top_p,min_p", [(0, 0.9, 0.0), (0, 1.0, 0.05), (5000, 0.5, 0.0)])
 def test_large_candidate_sets(hip, kind, n, top_k, top_p, min_p):
     rng = np.random.default_rng(n)
