@@ -298,6 +298,11 @@ __device__ __forceinline__ void sort_candidates(float *cval, uint32_t *cidx, uin
   }
 }
 
+// A candidate's logit as the list holds it: a NaN, which has no place in the
+// sort's order and could let an unused entry among the candidates, counts as
+// masked.
+__device__ __forceinline__ float list_logit(float v) { return v == v ? v : -INFINITY; }
+
 // Appends (v, i) of the lanes with `take` to the list, whatever its order
 // (the sort fixes it); *count may exceed kMaxCandidates, the excess is not
 // stored.
@@ -311,7 +316,7 @@ __device__ __forceinline__ void append(bool take, float v, uint32_t i, float *cv
   base = __shfl(base, lead, 64);
   const uint32_t at = base + (uint32_t)__popcll(m & ((1ull << lane) - 1));
   if (take && at < kMaxCandidates) {
-    cval[at] = v;
+    cval[at] = list_logit(v);
     cidx[at] = i;
   }
 }
@@ -626,12 +631,12 @@ __global__ __launch_bounds__(kSampleThreads) void k_sample(SampleArgs a) {
         const float v = logits[i];
         const uint32_t key = ord_key(v);
         if (kc >= n || key > prefix) {
-          cval[g] = v;
+          cval[g] = list_logit(v);
           cidx[g] = i;
           g++;
         } else if (key == prefix) {
           if (tot_gt + e < kc) {
-            cval[tot_gt + e] = v;
+            cval[tot_gt + e] = list_logit(v);
             cidx[tot_gt + e] = i;
           }
           e++;

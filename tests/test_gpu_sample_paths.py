@@ -96,3 +96,15 @@ def exact(x, top_k, top_p, min_p, temperature, u):
         lo, hi = np.searchsorted(c, u - 1e-4), np.searchsorted(c, u + 1e-4)
         found.update(keep[lo:hi + 1].tolist())
     return found
+
+
+@pytest.mark.parametrize("bits", [0x7fc00000, 0xffc00000, 0xffffffff], ids=hex)
+@pytest.mark.parametrize("n,top_k", [(100, 0), (100, 40), (5000, 40), (5000, 700), (5000, 1000), (5000, 0)])
+def test_nan_logits_draw_a_token(hip, n, top_k, bits):
+    """What a NaN makes of the weights is open, but the token is one of the
+    vocabulary: the next step reads its embedding row."""
+    rng = np.random.default_rng(n + top_k)
+    x = rng.standard_normal(n).astype(np.float32)
+    x.view(np.uint32)[rng.integers(0, n, 7)] = bits
+    for u in (0.0, 0.4, 0.999):
+        assert draw(hip, x, Sampling(0.8, top_k, 0.95, 0.05, 1.0), u) < n
