@@ -330,6 +330,9 @@ uint32_t attn_prefill_splits(uint32_t n_heads, uint32_t n_kv, uint32_t head_dim,
   // per split of the batch's middle tile, and no more partials than the
   // scratch holds.
   constexpr uint32_t kTargetGroups = 512, kMinSplitBlocks = 2, kMaxSplits = 16;
+  // A workgroup holds at most 128 rows (queries x heads), and several splits
+  // make fewer than 2·kTargetGroups workgroups.
+  static_assert(kAttnPartialFloats >= (2ull * kTargetGroups - 2) * 128 * (256 + 2), "the op's partials");
   const uint32_t per_wg = kPrefQ * attn_prefill_tiles(n_heads / n_kv);
   const uint32_t tiles = (n_queries + per_wg - 1) / per_wg;
   uint32_t want = (kTargetGroups + tiles * n_kv - 1) / (tiles * n_kv);
@@ -394,22 +397,11 @@ extern "C" int bch_attention_prefill(bch_ctx *ctx, bch_view q, bch_view k_cache,
   if (reinterpret_cast<uintptr_t>(kp) % 16 || reinterpret_cast<uintptr_t>(vp) % 16 ||
       reinterpret_cast<uintptr_t>(qp) % 16 || reinterpret_cast<uintptr_t>(op) % 16)
     return fail(BCH_ERR_ARGUMENT, "attention_prefill: operands must be 16-byte aligned");
-  // Key splits with their partials in the context's scratch; without the
-  // memory for them the launch runs unsplit.
-  float *partials = nullptr;
-  uint64_t partial_floats = 0;
-  const uint32_t splits = n_queries ? attn_prefill_splits(n_heads, n_kv_heads, head_dim, first_pos, n_queries, ~0ull) : 1;
-  if (splits > 1) {
-    void *p = nullptr;
-    partial_floats = attn_prefill_partial_floats(n_queries, n_heads, head_dim, splits);
-    if (ctx_scratch(ctx, partial_floats * 4, &p) == BCH_OK)
-      partials = static_cast<float *>(p);
-    else
-      (void)hipGetLastError();
-  }
+  // Key splits with their partials in memory that the context has held since
+  // it was opened (unsplit without it): a call allocates and waits for nothing.
   return launch(ctx, {"attention_prefill", 0, 0, 0}, [&](hipStream_t s) {
     run_attn_prefill_mfma(s, qp, kp, vp, op, n_heads, n_kv_heads, head_dim, first_pos, n_queries,
-                          n_heads * head_dim, n_heads * head_dim, 1.0f / sqrtf((float)head_dim), partials,
-                          partial_floats, nullptr, 0, 0);
+                          n_heads * head_dim, n_heads * head_dim, 1.0f / sqrtf((float)head_dim), ctx->attn_partials,
+                          ctx->attn_partials ? kAttnPartialFloats : 0, nullptr, 0, 0);
   });
 }

@@ -294,6 +294,8 @@ void run_attn_prefill_mfma(hipStream_t s, const float *q, const void *k_cache, c
 uint32_t attn_prefill_splits(uint32_t n_heads, uint32_t n_kv, uint32_t head_dim, uint32_t first_pos,
                              uint32_t n_queries, uint64_t partial_floats);
 // Floats of the partials of n_queries queries in `splits` key splits.
+// Partials of the most splits any launch takes on its own (heads of 256).
+constexpr uint64_t kAttnPartialFloats = 1022ull * 128 * 258;
 uint64_t attn_prefill_partial_floats(uint32_t n_queries, uint32_t n_heads, uint32_t head_dim, uint32_t splits);
 
 // matmul.hip.  Y[t] (store) W·X[t] for n_tokens rows; store 0 overwrite,

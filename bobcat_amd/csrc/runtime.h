@@ -43,6 +43,9 @@ struct bch_ctx {
   // Scratch of the op-level launchers (ctx_scratch), grown on demand.
   void *scratch = nullptr;
   uint64_t scratch_bytes = 0;
+  // Key-split partials of bch_attention_prefill (kAttnPartialFloats floats),
+  // from bch_open on; null if it could not have them.
+  float *attn_partials = nullptr;
 };
 
 namespace bch {

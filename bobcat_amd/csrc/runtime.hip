@@ -6,6 +6,7 @@
 #include <cstdio>
 #include <cstring>
 
+#include "kernels.h"
 #include "runtime.h"
 
 static thread_local std::string g_last_error;
@@ -111,6 +112,11 @@ int bch_open(bch_ctx **out) {
     delete ctx;
     return rc;
   }
+  // 129 MiB.  (Without them the prefill attention runs unsplit.)
+  if (hipMalloc(&ctx->attn_partials, kAttnPartialFloats * 4) != hipSuccess) {
+    (void)hipGetLastError();
+    ctx->attn_partials = nullptr;
+  }
   *out = ctx;
   return BCH_OK;
 }
@@ -125,6 +131,7 @@ void bch_close(bch_ctx *ctx) {
   if (ctx->begin_event) hipEventDestroy(ctx->begin_event);
   if (ctx->counters) hipFree(ctx->counters);
   if (ctx->scratch) hipFree(ctx->scratch);
+  if (ctx->attn_partials) hipFree(ctx->attn_partials);
   hipStreamDestroy(ctx->stream);
   delete ctx;
 }

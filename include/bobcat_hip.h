@@ -212,8 +212,8 @@ int bch_attention(bch_ctx *ctx, bch_view q, bch_view k_cache, bch_view v_cache, 
  * heads per KV head (else BCH_ERR_ATTENTION_LIMITS).  Queries and
  * probabilities enter the products as f16 high + low parts (~22 bits), so
  * results agree with bch_attention to ~1e-6 of the outputs' scale, not
- * bit for bit.  No scratch argument: the partials of its key splits (at
- * most ~140 MB) are the context's scratch, grown as bch_matmul grows it. */
+ * bit for bit.  No scratch: the partials of its key splits lie in 129 MiB
+ * that bch_open allocates, so a call allocates nothing and waits for nothing. */
 int bch_attention_prefill(bch_ctx *ctx, bch_view q, bch_view k_cache, bch_view v_cache, bch_view out,
                           uint32_t n_heads, uint32_t n_kv_heads, uint32_t head_dim, uint32_t first_pos,
                           uint32_t n_queries, uint32_t n_ctx);

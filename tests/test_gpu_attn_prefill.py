@@ -12,11 +12,13 @@ magnitude) instead of the op-level kernel's 1e-6.
 """
 from __future__ import annotations
 
+import ctypes as C
+
 import numpy as np
 import pytest
 
 from bobcat_amd import BobcatError
-from bobcat_amd.backend import attention_scratch_floats
+from bobcat_amd.backend import Hip, attention_scratch_floats
 
 pytestmark = pytest.mark.gpu
 
@@ -90,6 +92,31 @@ def test_attention_prefill_limits(hip):
             hip.attention_prefill(b.at(0), b.at(0), b.at(0), b.at(0), heads, kv_heads, dim, 0, 1, 16)
         hip.discard()
         assert e.value.status == ATTENTION_LIMITS
+
+
+def test_attention_prefill_allocates_nothing(hip):
+    """A context's first call with key splits leaves the device's free memory
+    as it was (the session's context has loaded the kernels)."""
+    runtime = C.CDLL("libamdhip64.so")
+
+    def free_bytes():
+        free, total = C.c_size_t(), C.c_size_t()
+        assert runtime.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        return free.value
+
+    heads, kv_heads, dim, first, queries = 32, 8, 64, 1536, 512
+    nbytes = (queries * heads * dim * 4, (first + queries) * kv_heads * dim * 2)
+    fresh = Hip()
+    try:
+        for ctx in (hip, fresh):
+            q, k, out = ctx.new_buffer(nbytes[0]), ctx.new_buffer(nbytes[1]), ctx.new_buffer(nbytes[0])
+            before = free_bytes()
+            run(ctx, lambda: ctx.attention_prefill(q.at(0), k.at(0), k.at(0), out.at(0), heads, kv_heads, dim, first,
+                                                   queries, first + queries))
+            after = free_bytes()
+    finally:
+        fresh.close()
+    assert after == before
 
 
 def test_attention_prefill_without_heads_writes_nothing(hip):
