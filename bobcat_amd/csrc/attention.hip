@@ -274,9 +274,15 @@ int bch_attention(bch_ctx *ctx, bch_view q, bch_view k_cache, bch_view v_cache, 
   if (reinterpret_cast<uintptr_t>(kp) % 16 || reinterpret_cast<uintptr_t>(vp) % 16)
     return fail(BCH_ERR_ARGUMENT, "attention: the caches must be 16-byte aligned");
   if (!ctx->counters) {
-    if (hipMalloc(&ctx->counters, kQueryBatch * 256 * 4) != hipSuccess)
+    void *p = nullptr;
+    if (hipMalloc(&p, kQueryBatch * 256 * 4) != hipSuccess)
       return fail(BCH_ERR_ALLOCATION, "attention: cannot allocate split counters");
-    hipMemset(ctx->counters, 0, kQueryBatch * 256 * 4);
+    // On the launches' own stream, which does not wait for the null stream.
+    if (hipMemsetAsync(p, 0, kQueryBatch * 256 * 4, ctx->stream) != hipSuccess) {
+      hipFree(p);
+      return fail(BCH_ERR_ALLOCATION, "attention: cannot clear split counters");
+    }
+    ctx->counters = static_cast<uint32_t *>(p);
   }
   if (n_kv_heads > 256) return fail(BCH_ERR_ATTENTION_LIMITS, "attention: at most 256 KV heads");
   return launch(ctx, {"attention", 0, 0, 0}, [&](hipStream_t s) {
