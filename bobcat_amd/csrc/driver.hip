@@ -546,6 +546,8 @@ int Sequence::restore(const void *blob, uint64_t bytes) {
     p += r.second;
   }
   BCH_TRY(check_hip(hipMemcpy(logits, p, (uint64_t)n_vocab * 4, hipMemcpyHostToDevice), "write logits"));
+  // (As after the weights' upload: the next step must not meet a copy in flight.)
+  BCH_TRY(check_hip(hipStreamSynchronize(nullptr), "write state"));
   n_past = saved_past;
   have_logits = have != 0;
   return BCH_OK;

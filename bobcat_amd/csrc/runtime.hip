@@ -159,9 +159,17 @@ int bch_buffer_new(bch_ctx *ctx, uint64_t len, bch_buffer **out) {
   return BCH_OK;
 }
 
+// Host memory to the device.  A copy from pageable memory may return before
+// its DMA has landed, and the contexts' (non-blocking) streams do not wait for
+// the null stream: a launch that follows must not start before the copy is done.
+static hipError_t copy_in(void *dst, const void *src, uint64_t bytes) {
+  const hipError_t e = hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice);
+  return e != hipSuccess ? e : hipStreamSynchronize(nullptr);
+}
+
 int bch_buffer_from_host(bch_ctx *ctx, const void *data, uint64_t len, bch_buffer **out) {
   BCH_TRY(bch_buffer_new(ctx, len, out));
-  if (len && hipMemcpy((*out)->ptr, data, len, hipMemcpyHostToDevice) != hipSuccess) {
+  if (len && copy_in((*out)->ptr, data, len) != hipSuccess) {
     bch_buffer_free(*out);
     *out = nullptr;
     return fail(BCH_ERR_ALLOCATION, "cannot copy %llu bytes to the device", (unsigned long long)len);
@@ -194,7 +202,7 @@ static int cpu_access(bch_ctx *ctx, bch_view view, uint64_t bytes, void **ptr) {
 int bch_write(bch_ctx *ctx, bch_view view, const void *data, uint64_t bytes) {
   void *p;
   BCH_TRY(cpu_access(ctx, view, bytes, &p));
-  if (bytes && hipMemcpy(p, data, bytes, hipMemcpyHostToDevice) != hipSuccess)
+  if (bytes && copy_in(p, data, bytes) != hipSuccess)
     return fail(BCH_ERR_EXECUTION, "host-to-device copy failed");
   return BCH_OK;
 }

@@ -1,6 +1,7 @@
 """CPU check of the host code's order on the device: the contexts' streams do
 not wait for the null stream, so a clear on it (hipMemset returns before it is
-done) is waited for before a launch can meet it."""
+done) or a copy on it from pageable memory (which may return once the bytes are
+staged) is waited for before a launch can meet it."""
 from __future__ import annotations
 
 import re
@@ -23,3 +24,7 @@ def unwaited(pattern: str) -> list[str]:
 
 def test_null_stream_clears_are_waited_for():
     assert unwaited(r"hipMemset\(") == []
+
+
+def test_null_stream_copies_to_the_device_are_waited_for():
+    assert unwaited(r"hipMemcpy\([^;]*hipMemcpyHostToDevice") == []
