@@ -555,14 +555,12 @@ extern "C" int bch_matmul_noalloc(bch_ctx *ctx, uint32_t format, bch_view weight
   if (store > 2) return fail(BCH_ERR_ARGUMENT, "matmul_noalloc: unknown store mode %u", store);
   if (n_rows == 0 || n_cols == 0 || n_cols % kBK)
     return fail(BCH_ERR_ARGUMENT, "matmul_noalloc: %u x %u needs columns in multiples of %d", n_rows, n_cols, kBK);
-  // The inputs plus the partials of the column split bch_matmul picks for
-  // this shape: when they fit, the launch below picks the same split (its
-  // smaller budget still holds it), so the results equal bch_matmul's bit
-  // for bit.
-  const GemmShape g = gemm_shape(format, n_rows, n_cols, n_tokens, (uint64_t)kMaxSplitK * n_tokens * n_rows, device_cus(),
-                                 false);
+  // The inputs plus the partials of the most column splits the shape may take
+  // (bch_matmul's pick is one of them, and with this much room the launch
+  // below picks the same, so the results equal bch_matmul's bit for bit).
+  const uint32_t most = gemm_max_splits(n_rows, n_cols, n_tokens, (uint64_t)kMaxSplitK * n_tokens * n_rows, device_cus());
   const uint64_t need = (matmul_split_bytes(n_tokens, n_cols) + 255) / 256 * 256 +
-                        (g.splits > 1 ? 4ull * g.splits * n_tokens * n_rows : 0);
+                        (most > 1 ? 4ull * most * n_tokens * n_rows : 0);
   if (need > kNoAllocScratchBytes)
     return fail(BCH_ERR_ARGUMENT,
                 "matmul_noalloc: %u tokens of %u x %u need %llu bytes of scratch, more than its %llu "

@@ -51,6 +51,18 @@ def test_binding_matches_header():
     assert not _lib.MISSING
 
 
+def test_noalloc_refuses_the_shapes_it_always_has():
+    """bch_matmul_noalloc's scratch is counted for the most column splits a
+    shape may take, whatever fewer the launch then picks: 4,630 x 10,240 at 651
+    tokens may take four, whose partials do not fit.  (Refused before the context
+    is looked at.)"""
+    from bobcat_amd import _lib
+
+    lib, none = _lib.lib(), _lib.View()
+    assert lib.bch_matmul_noalloc(None, 12, none, 4630, 10240, none, none, 651, 0) == 14  # Argument
+    assert b"bytes of scratch" in lib.bch_last_error()
+
+
 def test_row_bytes_and_scratch_sizes():
     from bobcat_amd import _lib
 
