@@ -352,8 +352,9 @@ static void lfm2_batch(bch_lfm2 *m, hipStream_t s, uint32_t pos, uint32_t count,
                    !pair_ok, L.up.data);
       } else if (!blas_pair) {
         run_matmul(s, L.gate.format, L.gate.data, m->n_ff, n, m->normed, m->ffn, count, 0, m->split, m->split_bytes,
-                   true);
+                   !pair_ok);
         check_finite(s, "gate", il, m->ffn, (uint64_t)count * m->n_ff);
+        // (The gate launch has left the inputs in the scratch.)
         run_matmul(s, L.up.format, L.up.data, m->n_ff, n, m->normed, m->ffn, count, 2, m->split, m->split_bytes, true);
       }
       check_finite(s, "swiglu", il, m->ffn, (uint64_t)count * m->n_ff);
