@@ -293,9 +293,9 @@ void run_attn_prefill_mfma(hipStream_t s, const float *q, const void *k_cache, c
 // (max, sum, output) partials going to `partials` (partial_floats floats).
 uint32_t attn_prefill_splits(uint32_t n_heads, uint32_t n_kv, uint32_t head_dim, uint32_t first_pos,
                              uint32_t n_queries, uint64_t partial_floats);
-// Floats of the partials of n_queries queries in `splits` key splits.
 // Partials of the most splits any launch takes on its own (heads of 256).
 constexpr uint64_t kAttnPartialFloats = 1022ull * 128 * 258;
+// Floats of the partials of n_queries queries in `splits` key splits.
 uint64_t attn_prefill_partial_floats(uint32_t n_queries, uint32_t n_heads, uint32_t head_dim, uint32_t splits);
 
 // matmul.hip.  Y[t] (store) W·X[t] for n_tokens rows; store 0 overwrite,
@@ -325,7 +325,8 @@ void finish_pending_sum(hipStream_t s, PendingSum &p, float *y);
 // receives that sum, written back to x; the pending sum is then cleared.
 // unscale_copy (optional, [rows]): for run_blas_pair, a second copy of the
 // token scales outside the scratch, and the fp16 inputs as plain rows (a
-// run_matmul that follows instead converts its own).
+// run_matmul that follows instead converts its own).  scratch null: the norm
+// alone (and the pending sum), for inputs that no run_matmul reads.
 void run_rms_norm_split(hipStream_t s, float *x, const float *w, float *out, uint32_t n, uint32_t rows, float eps,
                         void *scratch, PendingSum *pending = nullptr, float *unscale_copy = nullptr);
 // store 3: y = silu(W·x) ⊙ (W2·x), W and W2 the gate and up matrices of

@@ -315,7 +315,8 @@ static void lfm2_batch(bch_lfm2 *m, hipStream_t s, uint32_t pos, uint32_t count,
       check_finite(s, "attn_output", il, m->hidden, (uint64_t)count * n);
     }
     const bool pair_ok = L.gate_up16 && count > kBlasPairMinTokens;
-    run_rms_norm_split(s, m->hidden, L.ffn_norm, m->normed, n, count, m->norm_eps, m->split, &pend,
+    // (Experts take their inputs in grouped order and convert them themselves.)
+    run_rms_norm_split(s, m->hidden, L.ffn_norm, m->normed, n, count, m->norm_eps, L.moe ? nullptr : m->split, &pend,
                        pair_ok ? m->pair_us : nullptr);
     check_finite(s, "ffn_norm", il, m->normed, (uint64_t)count * n);
     if (L.moe) {

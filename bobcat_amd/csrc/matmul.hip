@@ -133,6 +133,7 @@ static void split_hi(hipStream_t s, const float *x, uint32_t rows, uint32_t frag
 // to x, exactly as k_gemm_reduce<1> would), and the sums are written back.
 //
 // rows_h: H gets plain rows (for the library GEMM) instead of fragments.
+// H null: the norm alone.
 template <int PER, int SPLITS>
 __global__ __launch_bounds__(256) void k_rms_norm_split(float *__restrict__ x, const float *__restrict__ w,
                                                        float *__restrict__ out, uint32_t n, float eps,
@@ -211,6 +212,7 @@ __global__ __launch_bounds__(256) void k_rms_norm_split(float *__restrict__ x, c
       mx = fmaxf(mx, fabsf(v));
     }
   }
+  if (!H) return;
   mx = block_max<256>(mx, red);
   int ex = 0;
   if (mx > 0.f) frexpf(mx, &ex);  // mx < 2^ex
@@ -245,12 +247,12 @@ void run_rms_norm_split(hipStream_t s, float *x, const float *w, float *out, uin
                         void *scratch, PendingSum *pending, float *unscale_copy) {
   if (!rows) return;
   _Float16 *hx = static_cast<_Float16 *>(scratch);
-  float *unscale = reinterpret_cast<float *>(hx + frag_halves(rows, n));
+  float *unscale = hx ? reinterpret_cast<float *>(hx + frag_halves(rows, n)) : nullptr;
   const bool rows_h = unscale_copy != nullptr;
   bool sum = pending && pending->splits > 1;
   const uint32_t ps = sum ? pending->splits : 0;
   if (sum && (pending->n != (uint64_t)rows * n || (ps != 2 && ps != 4 && ps != 8) ||
-              reinterpret_cast<const uint8_t *>(pending->part) < reinterpret_cast<uint8_t *>(unscale + rows))) {
+              (hx && reinterpret_cast<const uint8_t *>(pending->part) < reinterpret_cast<uint8_t *>(unscale + rows)))) {
     // Not this norm's rows, or the fp16 inputs written here would cover the
     // partials: add them first.
     finish_pending_sum(s, *pending, x);
