@@ -5,8 +5,6 @@
 
 namespace bch {
 
-typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
-
 // Fragment-major inputs: blocks of 32 tokens (the last holds the R that
 // remain, so nothing is padded), in a block [k / 8][token][k % 8].  Lane
 // l of a k-step of 16 columns reads 16 bytes: token l % 32, columns
@@ -16,17 +14,13 @@ __host__ __device__ __forceinline__ uint64_t frag_offset(uint32_t t, uint32_t k8
   return (uint64_t)b * 32 * n_cols + ((uint64_t)k8 * R + t % 32) * 8;
 }
 
-// Where a token's fp16 inputs go: halves 4·i4 .. of the token at
-// base + piece(i4).
+// Where a token's fp16 inputs go: columns 8i .. 8i+7 at base + i·stride.
 struct FragRow {
   _Float16 *base;
   uint32_t stride;  // halves between pieces of eight columns
   __device__ __forceinline__ static FragRow of(_Float16 *h, uint32_t t, uint32_t n_tokens, uint32_t n_cols) {
     const uint32_t b = t / 32;
     return {h + frag_offset(t, 0, n_tokens, n_cols), 8 * min(32u, n_tokens - 32 * b)};
-  }
-  __device__ __forceinline__ half4_t *quad(uint32_t i4) const {
-    return reinterpret_cast<half4_t *>(base + (uint64_t)(i4 / 2) * stride + 4 * (i4 % 2));
   }
   __device__ __forceinline__ _Float16 *at(uint32_t k) const { return base + (uint64_t)(k / 8) * stride + k % 8; }
 };
