@@ -8,10 +8,10 @@
 // has rows along the lanes and stores of 32 rows are contiguous).
 //
 // What bounds it: issue slots.  A wave issues an instruction every ~5 cycles
-// and a 32x32x16 MFMA occupies the matrix core for 33.6, so up to six other
-// instructions per MFMA are free (39.6 cycles with six, 60 with eight;
-// measured in registers alone), and there is no second wave on the SIMD to
-// hide more.  Hence:
+// and a 32x32x16 MFMA occupies the matrix core for 33.6: with six other
+// instructions beside it an MFMA takes 39.6 cycles, with eight 60 (measured in
+// registers alone), and there is no second wave on the SIMD to hide more.
+// Hence:
 //  * The inputs are stored fragment-major (frag_offset): each wave load is
 //    1 KB of consecutive bytes straight into MFMA operand registers.  Rows
 //    of tokens (32 cache lines per load) kept the L1 address path busy for
@@ -25,10 +25,12 @@
 //    group scheduling) left runs of a hundred instructions without an MFMA.
 //  * Every load has two to four stages to arrive and the LDS fragments of
 //    the next k-step are read one k-step ahead, across the barrier too.
-// 10752 x 2048 at 512 tokens: 33 us (715 TFLOP/s) against 51 for the kernel
-// this replaces (LDS rows, row-major inputs, a barrier that drained the
-// loads of every stage); 6144 x 2048: 19 against 31; 2048 x 2048 in two
-// splits: 9.9 against 17; 2048 x 10752 in four: 30 against 36 in eight.
+// 10752 x 2048 at 512 tokens: 34.3 us (657 TFLOP/s) against 50.4 for the
+// kernel this replaces (LDS rows, row-major inputs, a barrier that drained the
+// loads of every stage); 6144 x 2048: 21; 2048 x 10752 in four splits: 29.5
+// against 40.4 in eight.  A call with its input conversion and the sum of its
+// splits, before and after: 10752 x 2048 54.8 and 38.5 us, 6144 x 2048 35.4
+// and 25, 2048 x 2048 24.7 and 19.6, 2048 x 10752 55.2 and 43.
 #pragma once
 #include <type_traits>
 #include <utility>

@@ -86,7 +86,8 @@ __device__ __forceinline__ void split_row(uint32_t n8, FragRow row, float *unsca
 // Row t of X to fp16 fragments (split_row), one workgroup per row.  With
 // `entries`, row p of H is row entries[p] / x_div of X, at most last_row
 // (the positions of an expert-grouped launch).  Bound by the reads and the
-// scattered 16-byte writes: 512 x 10752 in 8.6 us.
+// scattered 16-byte writes: 512 x 10752 in 8.9 us (~6 when the inputs were
+// plain rows; the GEMM's loads gain more than that).
 template <int PER>
 __global__ __launch_bounds__(256) void k_split_hi(const float *__restrict__ X, uint32_t n_cols, uint32_t frag_rows,
                                                  const uint32_t *__restrict__ entries, uint32_t x_div, uint32_t last_row,
@@ -305,12 +306,15 @@ __global__ __launch_bounds__(256) void k_gemm_reduce(const float *__restrict__ P
 // plus 4 us to start and store), plus the partials' way through memory
 // (written and read at ~4.5 TB/s) and a launch to add them (half of its 2 us,
 // whether or not the next norm does it: the choice is the same for both, so
-// that both give the same bits).  So 6144 x 2048
-// at 512 tokens takes 64 x 256 tiles (192 of them, one round, 19 us; 28 with
-// 128 x 256 on 96 CUs), 10752 x 2048 takes 128 x 256 (33 us; 34 in two rounds
-// of 64 x 256), 3072 x 2048 takes 64 x 128, and 2048 x 10752 splits
-// its columns in four (30 us; 70 unsplit on 64 CUs, and eight splits of
-// 128 x 256 take as long but move twice the partials).
+// that both give the same bits).  What the choices give at 512 tokens, a
+// call with its input conversion and the sum of its splits, in us:
+//   6144 x 2048    64 x 256 (192 tiles, one round) 25; 64 x 128 26.6, 128 x 256 (96 CUs) 33
+//   10752 x 2048   128 x 256 37-38.5; 64 x 256 (two rounds) 38.5, 64 x 128 38.9
+//   3072 x 2048    64 x 128 18.3; 64 x 256 21, 128 x 256 31
+//   2048 x 10752   64 x 256 in four splits 43; 128 x 256 in eight 45.6 or four
+//                  50, 64 x 256 in eight 47, two 50 or unsplit (64 CUs) 77
+//   2048 x 2048    64 x 128 in two splits 19.6 (the driver's norms add them
+//                  on the way); unsplit 17.0, in four 25
 struct GemmShape {
   uint32_t mb, nb, splits;  // 32·mb rows x 128·nb tokens
 };
@@ -481,7 +485,11 @@ void run_matmul_experts(hipStream_t s, uint32_t format, const uint8_t *W, const 
   const HiInputs x{hx, unscale};
   const ExpertGroups g{offsets, entries, n_experts};
   // Tiles of 128 positions, or of 64 when the experts hold fewer: each tile
-  // converts its rows' weights again, and that is what bounds it.
+  // converts its rows' weights again, and that is what bounds it.  Pair and
+  // down of 1792 x 2048, 32 experts, 4 a token: at 40 positions an expert 62
+  // and 33 us with tiles of 64, 67 and 36 with 128; at 64 78 and 48, 74 and 41.
+  // The two cross, with tokens spread evenly at random, at 33 positions an
+  // expert of 128 experts, 46 of 64, 52 of 32 and 60 of 8.
   const bool few = positions <= 40 * n_experts;
   auto go = [&](auto fmt, auto mb, auto wr) {
     // 32·mb rows (half of them gate rows with `up`) x 128 / wr tokens.

@@ -23,7 +23,7 @@
 // (64 bytes a cycle, ~2 us per pass over 65,536 logits) and the latencies
 // between passes: loads are issued eight at a time, nothing is scanned by a
 // single thread, and the top-k path reads the logits twice (155 us before,
-// 29 us now for 65,536 logits, top-k 40; with top_k = 0 and top-p 0.9 a pass
+// 26 us now for 65,536 logits, top-k 40; with top_k = 0 and top-p 0.9 a pass
 // with its 8 us projection took 413 us and takes 189).
 // The draw comes from a wyrand generator whose 64-bit state lives in device
 // memory, so graph replays continue the stream.  Sums run as tree

@@ -241,9 +241,9 @@ uint64_t bch_attention_decode_scratch_floats(uint32_t n_heads, uint32_t head_dim
 
 /* bch_matmul without any allocation: the same kernels, column split and
  * results (bit for bit) as bch_matmul, with the launch's scratch — its fp16
- * inputs, n_tokens·(2·n_cols + 4) bytes, and the partial sums of the column
- * split bch_matmul picks for the shape, 4·splits·n_tokens·n_rows bytes when
- * it splits — in a static device array of bch_matmul_noalloc_max_bytes()
+ * inputs, n_tokens·(2·n_cols + 4) bytes, and the partial sums of the most
+ * column splits the shape may take, 4·splits·n_tokens·n_rows bytes if more
+ * than one — in a static device array of bch_matmul_noalloc_max_bytes()
  * (16 MiB) that each GPU holds for the life of the process, instead of
  * context scratch that may grow with hipMalloc.  No counterpart in the
  * reference: it is for callers that cannot allocate (code under HIP graph
